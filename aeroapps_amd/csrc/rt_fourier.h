@@ -1,5 +1,11 @@
 // Fourier-term kernels of the discrete-ordinate radiance path.
 //
+// Two paths per (streams, Stokes, precision) class (sym_path, rt_work.h).  The
+// symmetric path (k_pi, k_modes in rt_modes.h, k_adding in rt_adding.h) solves
+// symmetric eigenproblems and adds the layers; it takes n = N*S <= 12 in FP64
+// and n <= 7 mixed.  The general path below serves the larger classes and, item
+// by item (k_rescue), what the symmetric path hands over:
+//
 //   k_layer: one thread per (item, layer).  Homogeneous solutions
 //            (VLIDORT_QHOM_SOLUTION + ASYMTX, REG/vlidort_solutions.f90:150-1047,
 //            REG/vlidort_aux.f90:386-959), their normalisation
@@ -39,13 +45,15 @@
 #include "rt_work.h"
 #include "rt_device.h"
 #include "prof.h"
+#include "rt_converge.h"
+#include "rt_modes.h"
+#include "rt_adding.h"
 
 namespace aa {
 
 namespace {
 
 constexpr double DMS[4] = {1.0, 1.0, -1.0, -1.0};   // DMAT diagonal
-constexpr double VLIDORT_ACCURACY_D = (double)0.0001f;   // V283/VLIDORT_Mod.F90:232
 
 // Row slots of one band column live in up to five vectors of 8 doubles
 // (P##0..P##4).  With a wave-uniform slot index these macros compile to
@@ -99,8 +107,13 @@ __device__ __forceinline__ double dpp_d(double x) {
 }
 
 // ------------------------------------------------------------------ k_layer
+// Layer solution of one (item, layer) at Fourier term M on the general path:
+// SAB/DAB in srec, the layer record lrec and (bottom layer) the surface record
+// bbp are the item's.
 template <int N, int S, bool MIX>
-__global__ __launch_bounds__(64) void k_layer(RTWork W, int M) {
+__device__ __forceinline__ void layer_general(const RTWork& W, int M, int it, int layer,
+                                              const typename std::conditional<MIX, float, double>::type* srec,
+                                              double* lrec, double* bbp) {
   constexpr int n = N * S, LM = 2 * N;
   // MIX (the mixed path): SAB/DAB come from the FP32 MFMA contraction; from
   // N = 8 streams on, the source assembly -- the user-angle homogeneous
@@ -113,11 +126,7 @@ __global__ __launch_bounds__(64) void k_layer(RTWork W, int M) {
   using TR = typename std::conditional<MIX && (N >= 8), float, double>::type;
   constexpr LOff O(N, S);
   constexpr QOff QO(N, S);
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
   const int km = W.km;
-  if (t >= W.lcnt[M]) return;   // dense (item, layer) slots of this term
-  const int it = W.lown[t];
-  const int layer = t - W.loff[it];
   const int L = W.L_it[it];
   const int NMOM = W.nmoments;
   const double* __restrict__ Qt = W.quad;
@@ -152,10 +161,6 @@ __global__ __launch_bounds__(64) void k_layer(RTWork W, int M) {
   // contraction of every (item, layer) comes from the matrix-core kernel
   // k_sabdab (FP32 in the mixed path, FP64 otherwise); the diagonal term is
   // added here
-  using TSD = typename std::conditional<MIX, float, double>::type;
-  const TSD* srec;
-  if constexpr (MIX) srec = W.sab32 + il * (size_t)(2 * n * n);
-  else srec = W.sab64 + il * (size_t)(2 * n * n);
   double sab[n][n];
 #pragma unroll
   for (int i = 0; i < N; ++i) {
@@ -352,7 +357,6 @@ __global__ __launch_bounds__(64) void k_layer(RTWork W, int M) {
   // ---- layer record: X+-, transmittances and the homogeneous source
   // coefficients now; the beam solution's terms are written as they are
   // formed below (so that they hold no registers past their use)
-  double* lrec = W.lbuf + il * (size_t)W.lstride;
 #pragma unroll
   for (int i = 0; i < N; ++i)
 #pragma unroll
@@ -498,7 +502,7 @@ __global__ __launch_bounds__(64) void k_layer(RTWork W, int M) {
     if (W.bpdf && layer == L - 1) {
       constexpr BOff BO(N, n, S);
       constexpr BPOff PO(N);
-      double* bb = W.bbuf + (size_t)it * W.bstride;
+      double* bb = bbp;
       const double* rec = W.brdf + (size_t)it * W.brdf_stride;
       const double sfac = (M == 0) ? 2.0 : 1.0;
 #pragma unroll
@@ -558,7 +562,7 @@ __global__ __launch_bounds__(64) void k_layer(RTWork W, int M) {
     if (brdf || albedo != 0.0) {
       constexpr BOff BO(N, n, S);
       constexpr BROff RO(N);
-      double* bb = W.bbuf + (size_t)it * W.bstride;
+      double* bb = bbp;
       const double* rec = brdf ? W.brdf + (size_t)it * W.brdf_stride : nullptr;
       const double sfac = (M == 0) ? 2.0 : 1.0;
       const double kmult = 2.0 * albedo;
@@ -611,6 +615,20 @@ __global__ __launch_bounds__(64) void k_layer(RTWork W, int M) {
       }
     }
   }
+}
+
+template <int N, int S, bool MIX>
+__global__ __launch_bounds__(64) void k_layer(RTWork W, int M) {
+  constexpr int n = N * S;
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= W.lcnt[M]) return;   // dense (item, layer) slots of this term
+  const int it = W.lown[t];
+  const int layer = t - W.loff[it];
+  const size_t il = (size_t)it * W.km + layer;
+  double* lrec = W.lbuf + il * (size_t)W.lstride;
+  double* bb = W.bbuf + (size_t)it * W.bstride;
+  if constexpr (MIX) layer_general<N, S, MIX>(W, M, it, layer, W.sab32 + il * (size_t)(2 * n * n), lrec, bb);
+  else layer_general<N, S, MIX>(W, M, it, layer, W.sab64 + il * (size_t)(2 * n * n), lrec, bb);
 }
 
 // ------------------------------------------------------------------ k_bvp
@@ -695,10 +713,12 @@ __device__ __forceinline__ int grp_pivot(const bool (&eq)[SL], int g, int t, boo
   return (cmin == NONE) ? -1 : g * G + (cmin & 63);
 }
 
+// Boundary-value solve of Fourier term M for the wavefront's 64/G items (lane
+// group g holds item `it`; lbp, bb: its layer and surface records).  Returns,
+// on the group's lane 0, whether the item goes on to the next term.
 template <int N, int S, int G>
-__global__ __launch_bounds__(64, (N * S <= 6) ? 2 : 1) void k_bvp(RTWork W, int M, const int* __restrict__ active,
-                                            const int* __restrict__ nactive, int* __restrict__ next,
-                                            int* __restrict__ nnext) {
+__device__ __forceinline__ bool bvp_general(const RTWork& W, int M, int it, bool valid, const double* lbp, int LS,
+                                            const double* bb) {
   constexpr int n = N * S, n2 = 2 * n, NC = 4 * n, RH = NC, UW = NC + 2;
   constexpr int IPW = 64 / G, SL = bvp_slots(n, G);
   constexpr int NAC = (NC + G - 1) / G;   // accumulator columns per lane in the adjoint of the TOA recursion
@@ -719,27 +739,6 @@ __global__ __launch_bounds__(64, (N * S <= 6) ? 2 : 1) void k_bvp(RTWork W, int 
   const int lane = threadIdx.x, g = lane / G, t = lane - g * G;
   const unsigned long long gm = (G == 64) ? ~0ull : (((1ull << (G & 63)) - 1ull) << (g * G));
   const unsigned long long below = (1ull << lane) - 1ull;
-  // this wavefront's IPW items: the term's items are in LBINS lists by layer
-  // count, each list's wavefronts in turn
-  int first = -1, cntb = 0;
-  const int* lst = active;
-  {
-    int acc = 0;
-#pragma unroll
-    for (int b = 0; b < LBINS; ++b) {
-      const int c = nactive[b], nbk = (c + IPW - 1) / IPW;
-      if (first < 0 && (int)blockIdx.x < acc + nbk) {
-        first = ((int)blockIdx.x - acc) * IPW;
-        cntb = c;
-        lst = active + (size_t)b * W.cap;
-      }
-      acc += nbk;
-    }
-  }
-  if (first < 0) return;   // uniform over the wavefront
-  const int ai = first + g;
-  bool valid = ai < cntb;
-  const int it = valid ? lst[ai] : lst[first];
   const int km = W.km;
   const int gi = global_item(W, it), obs = gi / W.nch, ch = gi - obs * W.nch;
   const size_t oi = (size_t)ch * W.nobs + obs;
@@ -757,9 +756,10 @@ __global__ __launch_bounds__(64, (N * S <= 6) ? 2 : 1) void k_bvp(RTWork W, int 
   int Lmax = 0;
 #pragma unroll
   for (int q = 0; q < IPW; ++q) Lmax = max(Lmax, __builtin_amdgcn_readlane(L, q * G));
-  const int LS = W.lstride;
-  const double* __restrict__ lb = W.lbuf + (size_t)it * km * LS;
-  const double* __restrict__ bb = W.bbuf + (size_t)it * W.bstride;
+  // (not __restrict__: in k_rescue the records are written by the same kernel,
+  // and a load that the compiler takes for invariant may go through the scalar
+  // cache, which those writes do not reach)
+  const double* lb = lbp;
   constexpr BROff RO(N);
   constexpr BPOff PO(N);
   const bool brdf = W.brdf != nullptr;
@@ -1063,54 +1063,48 @@ __global__ __launch_bounds__(64, (N * S <= 6) ? 2 : 1) void k_bvp(RTWork W, int 
   // list and its (item, layer) slots, which the group's lanes then fill
   bool goes_on = false;
   if (t == 0 && valid) {
-    const double flux_multiplier = (M == 0) ? 1.0 : 2.0;
-    double* stk = W.stokes + (size_t)it * 3;
-    bool done = false;
     if (sing) {
       W.status[it] = 4;
       W.radiance[oi] = W.missing; W.reflectance[oi] = W.missing;
       if (S > 1) { W.qout[oi] = W.missing; W.uout[oi] = W.missing; }
       W.nfourier[oi] = 0;
     } else {
-      double sf[S];
-#pragma unroll
-      for (int o = 0; o < S; ++o) sf[o] = flux_multiplier * cum[o];
-      int testconv = W.testconv[it], fsaved = W.fsaved[it];
-      if (M == 0) {
-#pragma unroll
-        for (int o = 0; o < S; ++o) stk[o] = sf[o] + W.ss[(size_t)it * 3 + o] + W.db[(size_t)it * 3 + o];
-      } else {
-        const double azm = W.raa[obs] * (double)M * DEG_TO_RAD;
-        const double azmfac[3] = {cos(azm), cos(azm), sin(azm)};
-        double tazm[S], tnew[S];
-#pragma unroll
-        for (int o = 0; o < S; ++o) { tazm[o] = azmfac[o] * sf[o]; tnew[o] = stk[o] + tazm[o]; }
-        int count = 0;
-        if (tazm[0] != 0.0) { const double accur = fabs(tazm[0] / tnew[0]); if (accur < VLIDORT_ACCURACY_D) count++; }
-        else count++;
-#pragma unroll
-        for (int o = 0; o < S; ++o) stk[o] = tnew[o];
-        if (count == 1) {
-          testconv++;
-          if (testconv == 2) { done = true; fsaved = M; }
-        } else { testconv = 0; fsaved = 2 * N - 1; }
-      }
-      W.testconv[it] = testconv;
-      W.fsaved[it] = fsaved;
-      if (M >= W.nmoments) done = true;
-      if (done) {
-        const float pif = 4.0f * atanf(1.0f);
-        const double pi = (double)pif;
-        const double I = stk[0];
-        W.radiance[oi] = I;
-        W.reflectance[oi] = (pi * I) / (cos(W.sza[obs] * pi / (double)180.0f) * ff);
-        if (S > 1) { W.qout[oi] = stk[1]; W.uout[oi] = stk[2]; }
-        W.nfourier[oi] = fsaved + 1;
-      } else {
-        goes_on = true;
-      }
+      goes_on = converge_term<N, S>(W, it, obs, oi, ff, M, cum);
     }
   }
+  return goes_on;
+}
+
+template <int N, int S, int G>
+__global__ __launch_bounds__(64, (N * S <= 6) ? 2 : 1) void k_bvp(RTWork W, int M, const int* __restrict__ active,
+                                            const int* __restrict__ nactive, int* __restrict__ next,
+                                            int* __restrict__ nnext) {
+  constexpr int IPW = 64 / G;
+  const int lane = threadIdx.x, g = lane / G, t = lane - g * G;
+  // this wavefront's IPW items: the term's items are in LBINS lists by layer
+  // count, each list's wavefronts in turn
+  int first = -1, cntb = 0;
+  const int* lst = active;
+  {
+    int acc = 0;
+#pragma unroll
+    for (int b = 0; b < LBINS; ++b) {
+      const int c = nactive[b], nbk = (c + IPW - 1) / IPW;
+      if (first < 0 && (int)blockIdx.x < acc + nbk) {
+        first = ((int)blockIdx.x - acc) * IPW;
+        cntb = c;
+        lst = active + (size_t)b * W.cap;
+      }
+      acc += nbk;
+    }
+  }
+  if (first < 0) return;   // uniform over the wavefront
+  const int ai = first + g;
+  const bool valid = ai < cntb;
+  const int it = valid ? lst[ai] : lst[first];
+  const int L = valid ? W.L_it[it] : 0;
+  const bool goes_on = bvp_general<N, S, G>(W, M, it, valid, W.lbuf + (size_t)it * W.km * W.lstride, W.lstride,
+                                            W.bbuf + (size_t)it * W.bstride);
   const int noff = append_items(W, it, L, goes_on, nnext, next, W.lcnt + M + 1);
   const int goff = __builtin_amdgcn_ds_bpermute(4 * (lane - t), noff);
   if (goff >= 0)
@@ -1229,9 +1223,87 @@ __global__ __launch_bounds__(64) void k_sabdab(RTWork W, int M) {
   }
 }
 
-// One Fourier-term sweep with launch shapes (G lanes per item in k_bvp, PG
+// ------------------------------------------------------------------ k_rescue
+// The items that the symmetric path handed over (a layer without positive
+// definite S and D, a partially isolated eigenmatrix, a surface without
+// positive pivots): one wavefront takes an item through its remaining Fourier
+// terms on the general path, the layers across the lanes, then the band solve.
+// Launched once per chunk after the symmetric path's terms; the list is empty
+// for physical inputs and the launch then ends at once.
+template <int N, int S, bool MIX>
+__global__ __launch_bounds__(64) void k_rescue(RTWork W) {
+  constexpr int n = N * S, G = bvp_group(n);
+  constexpr YOff YO(N, S);
+  const int lane = threadIdx.x;
+  const int count = *W.rcnt, km = W.km, LS = LOff(N, S).size();
+  double* base = W.rbuf + (size_t)blockIdx.x * rescue_doubles(N, S, km);
+  double* lb = base + (size_t)km * (2 * n * n);
+  double* bb = lb + (size_t)km * LS;
+  for (int idx = blockIdx.x; idx < count; idx += gridDim.x) {
+    const int it = W.rlist[idx];
+    const int L = W.L_it[it];
+    for (int M = W.nfour[it] - 1; M <= W.nmoments; ++M) {
+      for (int layer = lane; layer < L; layer += 64) {
+        const double* og = W.og + ((size_t)it * km + layer) * (size_t)YO.K;
+        using T = typename std::conditional<MIX, float, double>::type;
+        T* srec = reinterpret_cast<T*>(base + (size_t)layer * (2 * n * n));
+        const T* Y;
+        if constexpr (MIX) Y = W.ytab;
+        else Y = W.ytab64;
+#pragma unroll 1
+        for (int r = 0; r < YO.rows(); ++r) {
+          T v = (T)0;
+#pragma unroll 1
+          for (int q = 0; q < YO.K; ++q) v += Y[YO.at(M, r, q)] * (T)og[q];
+          srec[r] = v;
+        }
+        layer_general<N, S, MIX>(W, M, it, layer, srec, lb + (size_t)layer * LS, bb);
+      }
+      __threadfence_block();
+      const bool on = bvp_general<N, S, G>(W, M, it, lane < G, lb, LS, bb);
+      __threadfence_block();
+      if (__ballot(lane == 0 && on) == 0ull) break;
+    }
+  }
+}
+
+// The Fourier terms of a chunk on the symmetric path.
+template <int N, int S, bool MIX, int PG>
+int fourier_loop_sym(const RTWork& W, int nitems, int* const lists[2], int* counts, hipStream_t st) {
+  const int nl = (int)(((size_t)nitems * W.km + 63) / 64);
+  const int ns = (int)(((size_t)nitems * W.km + 16 * PG - 1) / (16 * PG));
+  const int nb = (nitems + 3) / 4 + LBINS;
+  prof_begin(PROF_ITEM, st);
+  hipLaunchKernelGGL((k_pi<N, S>), dim3((unsigned)(((size_t)nitems * 2 * N + 63) / 64)), dim3(64), 0, st, W, nitems);
+  prof_end(PROF_ITEM, st);
+  for (int M = 0; M <= W.nmoments; ++M) {
+    const int* in = lists[M & 1];
+    int* out = lists[(M + 1) & 1];
+    if constexpr (needs_sabdab(N, S, MIX)) {
+      prof_begin(PROF_SABDAB, st);
+      hipLaunchKernelGGL((k_sabdab<N, S, typename std::conditional<MIX, float, double>::type, PG>), dim3(ns), dim3(64),
+                         0, st, W, M);
+      prof_end(PROF_SABDAB, st);
+    }
+    prof_begin(PROF_LAYER, st);
+    hipLaunchKernelGGL((k_modes<N, S, MIX>), dim3(nl), dim3(64), 0, st, W, M);
+    prof_end(PROF_LAYER, st);
+    prof_begin(PROF_BVP, st);
+    hipLaunchKernelGGL((k_adding<N, S, MIX>), dim3(nb), dim3(64), 0, st, W, M, in, counts + M * LBINS, out,
+                       counts + (M + 1) * LBINS);
+    prof_end(PROF_BVP, st);
+    if (W.mid_event && M == std::min(W.mid_term, W.nmoments)) AA_CHECK(hipEventRecord(W.mid_event, st));
+  }
+  prof_begin(PROF_BVP, st);
+  hipLaunchKernelGGL((k_rescue<N, S, MIX>), dim3(W.rblocks), dim3(64), 0, st, W);
+  prof_end(PROF_BVP, st);
+  AA_CHECK(hipGetLastError());
+  return 0;
+}
+
+// One Fourier-term sweep on the general path with launch shapes (G lanes per item in k_bvp, PG
 // 16-pair groups per wavefront in k_sabdab); every shape gives the same bits.
-template <int N, int S, int G, int PG>
+template <int N, int S, bool MIX, int G, int PG>
 int fourier_loop_shape(const RTWork& W, int nitems, int* const lists[2], int* counts, hipStream_t st) {
   const int nl = (int)(((size_t)nitems * W.km + 63) / 64);
   const int ns = (int)(((size_t)nitems * W.km + 16 * PG - 1) / (16 * PG));
@@ -1240,12 +1312,11 @@ int fourier_loop_shape(const RTWork& W, int nitems, int* const lists[2], int* co
     const int* in = lists[M & 1];
     int* out = lists[(M + 1) & 1];
     prof_begin(PROF_SABDAB, st);
-    if (W.precision == 1) hipLaunchKernelGGL((k_sabdab<N, S, float, PG>), dim3(ns), dim3(64), 0, st, W, M);
-    else hipLaunchKernelGGL((k_sabdab<N, S, double, PG>), dim3(ns), dim3(64), 0, st, W, M);
+    hipLaunchKernelGGL((k_sabdab<N, S, typename std::conditional<MIX, float, double>::type, PG>), dim3(ns), dim3(64), 0,
+                       st, W, M);
     prof_end(PROF_SABDAB, st);
     prof_begin(PROF_LAYER, st);
-    if (W.precision == 1) hipLaunchKernelGGL((k_layer<N, S, true>), dim3(nl), dim3(64), 0, st, W, M);
-    else hipLaunchKernelGGL((k_layer<N, S, false>), dim3(nl), dim3(64), 0, st, W, M);
+    hipLaunchKernelGGL((k_layer<N, S, MIX>), dim3(nl), dim3(64), 0, st, W, M);
     prof_end(PROF_LAYER, st);
     prof_begin(PROF_BVP, st);
     hipLaunchKernelGGL((k_bvp<N, S, G>), dim3(nb), dim3(64), 0, st, W, M, in, counts + M * LBINS, out,
@@ -1258,17 +1329,29 @@ int fourier_loop_shape(const RTWork& W, int nitems, int* const lists[2], int* co
 }
 
 // The launch shapes of W.shape_bvp / W.shape_sab (0: default, 1: the
-// alternative the tuner may pick).
-template <int N, int S>
-int fourier_loop(const RTWork& W, int nitems, int* const lists[2], int* counts, hipStream_t st) {
+// alternative the tuner may pick); the band solver's shapes exist on the
+// general path only.
+template <int N, int S, bool MIX>
+int fourier_loop_prec(const RTWork& W, int nitems, int* const lists[2], int* counts, hipStream_t st) {
   constexpr int n = N * S;
-  constexpr int G0 = bvp_group(n), G1 = bvp_group_alt(n);
   constexpr int P0 = sab_groups(N, S), P1 = sab_groups_alt(N, S);
   const bool gb = W.shape_bvp == 1, gs = W.shape_sab == 1;
-  if (!gb && !gs) return fourier_loop_shape<N, S, G0, P0>(W, nitems, lists, counts, st);
-  if (gb && !gs) return fourier_loop_shape<N, S, G1, P0>(W, nitems, lists, counts, st);
-  if (!gb && gs) return fourier_loop_shape<N, S, G0, P1>(W, nitems, lists, counts, st);
-  return fourier_loop_shape<N, S, G1, P1>(W, nitems, lists, counts, st);
+  if constexpr (sym_path(N, S, MIX)) {
+    if (gs) return fourier_loop_sym<N, S, MIX, P1>(W, nitems, lists, counts, st);
+    return fourier_loop_sym<N, S, MIX, P0>(W, nitems, lists, counts, st);
+  } else {
+    constexpr int G0 = bvp_group(n), G1 = bvp_group_alt(n);
+    if (!gb && !gs) return fourier_loop_shape<N, S, MIX, G0, P0>(W, nitems, lists, counts, st);
+    if (gb && !gs) return fourier_loop_shape<N, S, MIX, G1, P0>(W, nitems, lists, counts, st);
+    if (!gb && gs) return fourier_loop_shape<N, S, MIX, G0, P1>(W, nitems, lists, counts, st);
+    return fourier_loop_shape<N, S, MIX, G1, P1>(W, nitems, lists, counts, st);
+  }
+}
+
+template <int N, int S>
+int fourier_loop(const RTWork& W, int nitems, int* const lists[2], int* counts, hipStream_t st) {
+  if (W.precision == 1) return fourier_loop_prec<N, S, true>(W, nitems, lists, counts, st);
+  return fourier_loop_prec<N, S, false>(W, nitems, lists, counts, st);
 }
 
 }  // namespace

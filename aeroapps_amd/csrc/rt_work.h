@@ -88,7 +88,7 @@ struct RTWork {
   int* beam_cutoff = nullptr;
   int* testconv = nullptr;
   int* fsaved = nullptr;
-  int* nfour = nullptr;            // Fourier terms done
+  int* nfour = nullptr;            // 0, or 1 + the Fourier term at which k_rescue takes the item up
   // the active (item, layer) pairs of the current Fourier term, numbered
   // densely: item it owns slots loff[it] .. loff[it] + L - 1, lown[slot] = it;
   // lcnt[M] is the number of slots of term M (filled where the term's item
@@ -120,11 +120,23 @@ struct RTWork {
   double* tr = nullptr;            // [it][km][TR_NFIELDS]
   double* lev = nullptr;           // [it][km+1][4]: tauslant, suntau, atten, FO mult(enhanced)
   double* lostrans = nullptr;      // [it][km+1]
+  // symmetric path (k_modes, k_adding)
+  double* abuf = nullptr;          // [it][km][astride] layer modes (AOff)
+  double* pis = nullptr;           // [it][PiOff] PI functions of the user angle and the solar cosine
+  int astride = 0;
+  // general path (k_layer, k_bvp)
   double* lbuf = nullptr;          // [it][km][lstride] homogeneous + particular solutions
   double* bbuf = nullptr;          // [it][bstride] surface terms of the bottom layer
   int lstride = 0, bstride = 0;
+  // items of the symmetric path that continue on the general path (k_rescue):
+  // list, count, and one item's records per workgroup
+  int* rlist = nullptr;
+  int* rcnt = nullptr;
+  int rblocks = 0;
+  double* rbuf = nullptr;          // [rblocks][rescue_doubles]
   // ---- quadrature and PI tables of the quadrature streams (device)
-  const double* quad = nullptr;    // [qs N][qw N][xq: M][l][i][S][S]
+  const double* quad = nullptr;    // QOff: [qs N][qw N][xq: M][l][i][S][S][scalings]
+  const double* phi = nullptr;     // the same layout, xq times sqrt(w_i/mu_i)
   // ---- mixed precision: FP32 phase-matrix contraction (SAB/DAB) by MFMA
   int precision = 0;               // 0 FP64, 1 mixed
   const float* ytab = nullptr;     // [M][2n^2 rows][2N*S*S] contraction weights
@@ -168,6 +180,51 @@ struct LOff {
   __host__ __device__ constexpr int csrc(int o) const { return 2 * n * n + 5 * n + 2 * n * S + o; }
   __host__ __device__ constexpr int size() const { return (2 * n * n + 5 * n + 2 * n * S + S + 1) & ~1; }
 };
+
+// Offsets inside one abuf record (per item and layer) of the symmetric path,
+// n = N*S: the modes' sum and difference vectors E(r, k), F(r, k) in the
+// scaled streams, the layer transmittances and beam amplitudes of the modes,
+// the coefficients of the upwelling source at the user angle (of the
+// down-decaying and up-decaying amplitudes) and its beam part.
+struct AOff {
+  int n, S;
+  __host__ __device__ constexpr AOff(int N_, int S_) : n(N_ * S_), S(S_) {}
+  __host__ __device__ constexpr int e(int r, int k) const { return r * n + k; }
+  __host__ __device__ constexpr int f(int r, int k) const { return n * n + r * n + k; }
+  __host__ __device__ constexpr int t(int k) const { return 2 * n * n + k; }
+  __host__ __device__ constexpr int gup(int k) const { return 2 * n * n + n + k; }
+  __host__ __device__ constexpr int gdn(int k) const { return 2 * n * n + 2 * n + k; }
+  __host__ __device__ constexpr int cl(int o, int k) const { return 2 * n * n + 3 * n + o * n + k; }
+  __host__ __device__ constexpr int cm(int o, int k) const { return 2 * n * n + 3 * n + (S + o) * n + k; }
+  __host__ __device__ constexpr int csrc(int o) const { return 2 * n * n + 3 * n + 2 * S * n + o; }
+  __host__ __device__ constexpr int size() const { return (2 * n * n + 3 * n + 2 * S * n + S + 1) & ~1; }
+};
+
+// Offsets inside one item's PI record: functions p (P; P, R, T with three
+// Stokes components) of degree l and Fourier term M at the user angle (w = 0)
+// and the solar cosine (w = 1).
+struct PiOff {
+  int LM, P;
+  __host__ __device__ constexpr PiOff(int N_, int S_) : LM(2 * N_), P(S_ == 1 ? 1 : 3) {}
+  __host__ __device__ constexpr int at(int M, int l, int w, int p) const { return ((M * LM + l) * 2 + w) * P + p; }
+  __host__ __device__ constexpr int size() const { return LM * LM * 2 * P; }
+};
+
+// Whether a (streams, Stokes, precision) class runs on the symmetric path.
+// FP64: n = N*S <= 12, where the Jacobi iteration's matrix (2 n^2 registers)
+// still fits the register file of a lane.  Mixed: n <= 7, where E and F fit
+// together (the perturbation step mixes their columns); from N = 8 on the
+// mixed path's FP32 source assembly belongs to k_layer.
+constexpr int SYM_MAX_N = 12, SYM_MAX_N_MIXED = 7;
+__host__ __device__ constexpr bool sym_path(int N, int S, bool mixed) {
+  return N * S <= (mixed ? SYM_MAX_N_MIXED : SYM_MAX_N);
+}
+// SAB/DAB from k_sabdab: always in the mixed path, with three Stokes
+// components, and on the general path (the symmetric scalar FP64 path forms
+// the two triangles in k_modes).
+__host__ __device__ constexpr bool needs_sabdab(int N, int S, bool mixed) {
+  return mixed || S != 1 || !sym_path(N, S, mixed);
+}
 
 // Offsets inside one bbuf record: surface reflection terms of the bottom
 // layer for the current Fourier term, per quadrature row i < N (the
@@ -262,9 +319,19 @@ struct QOff {
   __host__ __device__ constexpr int xq(int M, int l, int i, int s1, int s2) const {
     return 2 * N + ((((M * 2 * N + l) * N + i) * S + s1) * S + s2);
   }
-  __host__ __device__ constexpr int size() const { return 2 * N + 2 * N * 2 * N * N * S * S; }
+  // scalings of stream i: sqrt(w mu), its inverse, 1 / mu
+  __host__ __device__ constexpr int g(int i) const { return 2 * N + 2 * N * 2 * N * N * S * S + i; }
+  __host__ __device__ constexpr int rg(int i) const { return 3 * N + 2 * N * 2 * N * N * S * S + i; }
+  __host__ __device__ constexpr int rmu(int i) const { return 4 * N + 2 * N * 2 * N * N * S * S + i; }
+  __host__ __device__ constexpr int size() const { return 5 * N + 2 * N * 2 * N * N * S * S; }
 };
 
+
+// Doubles of one workgroup's records in k_rescue: SAB/DAB, layer solutions and
+// surface terms of one item.
+__host__ __device__ constexpr size_t rescue_doubles(int N, int S, int km) {
+  return (size_t)km * (2 * N * S * N * S + LOff(N, S).size()) + BOff(N, N * S, S).size();
+}
 
 // Launch shapes of the Fourier-term kernels.  Lanes per item of the band
 // solver: 8 for n = N*S <= 8 (8 items per wavefront), the smallest power of

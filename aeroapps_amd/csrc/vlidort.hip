@@ -159,7 +159,12 @@ void quad_table_t(int N, int nmoments, std::vector<double>& q) {
   std::vector<double> qs(N), qw(N);
   if (N == 1) { qs[0] = std::sqrt(1.0 / 3.0); qw[0] = 1.0; }
   else getquad2(0.0, 1.0, N, qs.data(), qw.data());
-  for (int i = 0; i < N; ++i) { q[QO.qs(i)] = qs[i]; q[QO.qw(i)] = qw[i]; }
+  for (int i = 0; i < N; ++i) {
+    q[QO.qs(i)] = qs[i]; q[QO.qw(i)] = qw[i];
+    q[QO.g(i)] = std::sqrt(qw[i] * qs[i]);
+    q[QO.rg(i)] = 1.0 / q[QO.g(i)];
+    q[QO.rmu(i)] = 1.0 / qs[i];
+  }
   for (int M = 0; M < LM; ++M) {
     if (M > nmoments) break;
     for (int i = 0; i < N; ++i) {
@@ -223,6 +228,18 @@ const std::vector<double>& quad_table_cached(int N, int S, int nmoments) {
   if (it == cache.end()) {
     std::vector<double> q;
     quad_table(N, S, nmoments, q);
+    // the symmetric path's copy: PI matrices scaled by sqrt(w_i / mu_i)
+    QOff QO(N, S);
+    const size_t sz = (size_t)QO.size();
+    q.resize(2 * sz, 0.0);
+    for (int M = 0; M < 2 * N; ++M)
+      for (int l = 0; l < 2 * N; ++l)
+        for (int i = 0; i < N; ++i)
+          for (int a = 0; a < S; ++a)
+            for (int b = 0; b < S; ++b) {
+              const int k = QO.xq(M, l, i, a, b);
+              q[sz + k] = std::sqrt(q[QO.qw(i)] / q[QO.qs(i)]) * q[k];
+            }
     it = cache.emplace(key, std::move(q)).first;
   }
   return it->second;
@@ -326,20 +343,34 @@ size_t carve_work(Carver& C, RTWork& W, int cap) {
   W.tr = C.take<double>((size_t)cap * km * TR_NFIELDS);
   W.lev = C.take<double>((size_t)cap * (km + 1) * 4);
   W.lostrans = C.take<double>((size_t)cap * (km + 1));
-  W.lbuf = C.take<double>((size_t)cap * km * W.lstride);
-  W.bbuf = C.take<double>((size_t)cap * W.bstride);
+  const bool mixed = W.precision == 1;
+  const bool sym = sym_path(W.N, W.S, mixed);
+  W.astride = AOff(W.N, W.S).size();
+  if (sym) {
+    W.abuf = C.take<double>((size_t)cap * km * W.astride);
+    W.pis = C.take<double>((size_t)cap * PiOff(W.N, W.S).size());
+    W.rlist = C.take<int>(cap);
+    // workgroups of k_rescue: up to 512, fewer for small chunks, so that their
+    // records add at most an eighth of an item's general-path records to each item
+    W.rblocks = std::min(512, (cap + 7) / 8);
+    W.rbuf = C.take<double>((size_t)W.rblocks * rescue_doubles(W.N, W.S, km));
+  } else {
+    W.lbuf = C.take<double>((size_t)cap * km * W.lstride);
+    W.bbuf = C.take<double>((size_t)cap * W.bstride);
+  }
   W.brdf = (W.kernel_wt || W.u10m || W.bpdf) ? C.take<double>((size_t)cap * W.brdf_stride) : nullptr;
   W.wsa_cache = W.kernel_wt ? C.take<double>(4) : nullptr;
-  W.sab32 = (W.precision == 1) ? C.take<float>((size_t)cap * km * 2 * n * n) : nullptr;
-  W.sab64 = (W.precision == 0) ? C.take<double>((size_t)cap * km * 2 * n * n) : nullptr;
+  W.sab32 = mixed ? C.take<float>((size_t)cap * km * 2 * n * n) : nullptr;
+  W.sab64 = (!mixed && needs_sabdab(W.N, W.S, mixed)) ? C.take<double>((size_t)cap * km * 2 * n * n) : nullptr;
   return C.off;
 }
 
 size_t bytes_per_item(const RTWork& W0) {
   RTWork W = W0;
+  // (8 items share one rescue workgroup)
   Carver a(nullptr), b(nullptr);
-  size_t s1 = carve_work(a, W, 1), s2 = carve_work(b, W, 2);
-  return s2 - s1 + 256 * 24;
+  size_t s1 = carve_work(a, W, 8), s2 = carve_work(b, W, 16);
+  return (s2 - s1 + 7) / 8 + 256 * 24;
 }
 
 // Items of one work chunk of W's shape on the current GPU: the work budget
@@ -399,8 +430,9 @@ int run_items(RTWork W, int g0, int g1, hipStream_t st, const int* d_items = nul
   size_t capi = 1;
   const size_t tab_bytes = qtab.size() * sizeof(double) + std::max<size_t>(1, ytab.size()) * sizeof(float) +
                            std::max<size_t>(1, ytab64.size()) * sizeof(double) +
-                           std::max<size_t>(1, btab.size()) * sizeof(double) + sizeof(int) * (W.nmoments + 2) +
-                           16 * 256;
+                           std::max<size_t>(1, btab.size()) * sizeof(double) +
+                           sizeof(int) * ((LBINS + 1) * (W.nmoments + 2) + 1) +
+                           rescue_doubles(W.N, W.S, W.km) * sizeof(double) + 16 * 256;
   if (fixed_base) {
     const size_t per = bytes_per_item(W) + 2 * LBINS * sizeof(int);
     if (fixed_bytes <= tab_bytes + per) return AA_EDIMS;
@@ -424,8 +456,9 @@ int run_items(RTWork W, int g0, int g1, hipStream_t st, const int* d_items = nul
     dbt = C.take<double>(std::max<size_t>(1, btab.size()));
     *l0 = C.take<int>((size_t)LBINS * cap);
     *l1 = C.take<int>((size_t)LBINS * cap);
-    // per Fourier term: items of each layer-count list, then (item, layer) slots
-    *cnt = C.take<int>((LBINS + 1) * (W.nmoments + 2));
+    // per Fourier term: items of each layer-count list, then (item, layer) slots;
+    // last the count of k_rescue's list
+    *cnt = C.take<int>((LBINS + 1) * (W.nmoments + 2) + 1);
     return C.off;
   };
   double* dq; int *l0, *l1, *cnt;
@@ -440,6 +473,7 @@ int run_items(RTWork W, int g0, int g1, hipStream_t st, const int* d_items = nul
   carve_all(base, W, &dq, &l0, &l1, &cnt);
   AA_CHECK(hipMemcpyAsync(dq, qtab.data(), qtab.size() * sizeof(double), hipMemcpyHostToDevice, st));
   W.quad = dq;
+  W.phi = dq + QOff(W.N, W.S).size();
   if (!ytab.empty()) {
     AA_CHECK(hipMemcpyAsync(dy, ytab.data(), ytab.size() * sizeof(float), hipMemcpyHostToDevice, st));
     W.ytab = dy;
@@ -455,10 +489,11 @@ int run_items(RTWork W, int g0, int g1, hipStream_t st, const int* d_items = nul
   int* lists[2] = {l0, l1};
   W.item_list = d_items;
   W.lcnt = cnt + LBINS * (W.nmoments + 2);
+  W.rcnt = cnt + (LBINS + 1) * (W.nmoments + 2);
   for (int item0 = g0; item0 < g1; item0 += cap) {
     const int ni = std::min(cap, g1 - item0);
     W.item0 = item0;
-    AA_CHECK(hipMemsetAsync(cnt, 0, sizeof(int) * (LBINS + 1) * (W.nmoments + 2), st));
+    AA_CHECK(hipMemsetAsync(cnt, 0, sizeof(int) * ((LBINS + 1) * (W.nmoments + 2) + 1), st));
     if (rt_setup(W, ni, lists[0], cnt, st)) return AA_EHIP;
     int e = rt_fourier(W, ni, lists, cnt, st);
     if (e) return e == -4 ? AA_EDIMS : AA_EHIP;
