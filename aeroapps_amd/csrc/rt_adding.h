@@ -37,6 +37,7 @@
 #include <type_traits>
 #include "rt_work.h"
 #include "rt_device.h"
+#include "rt_modes.h"
 
 namespace aa {
 
@@ -47,15 +48,6 @@ template <int K>
 __device__ __forceinline__ double bc16(double x) {
   return __builtin_amdgcn_update_dpp(x, x, 0x150 + K, 0xF, 0xF, true);
 }
-// compile-time loop: f(integral_constant<int, B>) .. f(integral_constant<int, E - 1>)
-template <int B, int E, class F>
-__device__ __forceinline__ void static_for(F&& f) {
-  if constexpr (B < E) {
-    f(std::integral_constant<int, B>());
-    static_for<B + 1, E>(f);
-  }
-}
-
 // Solves K X = X in place (lane c: column c of K and of the right-hand sides),
 // Gaussian elimination without row exchanges.  `low` collects the smallest
 // pivot.
@@ -143,7 +135,7 @@ __global__ __launch_bounds__(64) void k_adding(RTWork W, int M, const int* __res
 #pragma unroll
   for (int q = 0; q < IPW; ++q) Lmax = max(Lmax, __builtin_amdgcn_readlane(L, q * 16));
   const int AS = W.astride;
-  const double* __restrict__ ab = W.abuf + (size_t)it * km * AS;
+  const double* __restrict__ ab = W.abuf + (size_t)W.loff[it] * AS;   // the item's slots of this term
   const double* __restrict__ trr = W.tr + (size_t)it * km * TR_NFIELDS;
   const double* __restrict__ Qt = W.quad;
   const double ff = W.flux ? W.flux[(size_t)obs * W.nch + ch] : 1.0;
@@ -159,7 +151,7 @@ __global__ __launch_bounds__(64) void k_adding(RTWork W, int M, const int* __res
     const int c = col ? t : 0;
 #pragma unroll
     for (int m = 0; m < n; ++m) {
-      const double x = r[O.e(m, 0) + c], y = r[O.f(m, 0) + c];
+      const double x = r[O.e(m, 0) + c * O.estep()], y = r[O.f(m, 0) + c * O.estep()];
       e[m] = col ? x : 0.0;
       f[m] = col ? y : 0.0;
     }

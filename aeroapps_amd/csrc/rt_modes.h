@@ -42,8 +42,11 @@
 // error is the square of 1e-7.
 //
 // Measured against k_layer + k_sabdab (per call): N = 6 FP64, 400,000 items
-// 201 -> 127 ms; N = 12, 1,200 items 32.8 -> 4.9 ms; three Stokes components
-// N = 4, 16,000 items 361 -> 71 ms (with k_sabdab).
+// 201 -> 59 ms (127 with the records stored straight from the lanes), mixed,
+// 240,004 items 110 -> 63 ms (168); N = 12, 1,200 items 32.8 -> 2.8 ms (4.9);
+// three Stokes components N = 4, 16,000 items 361 -> 45 ms (71; 12 of them
+// k_sabdab).  At N = 6 the records are written at 2.1 TB/s and the VALU issues
+// 5.5k instructions per wavefront.
 #pragma once
 #include <type_traits>
 #include "rt_work.h"
@@ -69,6 +72,15 @@ __device__ __forceinline__ double rsqrt_nr(double x) {
   h = 0.5 * y;
   e = fma(-x * y, h, 0.5);
   return fma(y, e, y);
+}
+
+// compile-time loop: f(integral_constant<int, B>) .. f(integral_constant<int, E - 1>)
+template <int B, int E, class F>
+__device__ __forceinline__ void static_for(F&& f) {
+  if constexpr (B < E) {
+    f(std::integral_constant<int, B>());
+    static_for<B + 1, E>(f);
+  }
 }
 
 // PI functions of every Fourier term: one thread per (item, M).
@@ -131,21 +143,58 @@ __device__ __forceinline__ bool cholesky(double (&a)[n * (n + 1) / 2]) {
   return ok;
 }
 
+// A wavefront's records go to memory through LDS: every lane puts the fields of
+// its record in order, and each 64-byte piece is written whole, eight records
+// per store.  Stored from the lanes directly (8 bytes of 64 records per store,
+// 13 MB of records open at once against 4 MB of L2) the pieces were evicted
+// partially written: 53 GB for 12 GB of records (N = 6, 40,022 items), which
+// bounded the kernel.
+struct RecordOut {
+  double* base;       // the wavefront's first record
+  int left, lane;     // records of the wavefront, this lane
+  double (*lds)[9];   // [64][8 + 1]
+  template <int f, int AS>
+  __device__ __forceinline__ void put(double v) {
+    lds[lane][f & 7] = v;
+    if constexpr ((f & 7) == 7) flush<f & ~7, AS>();
+  }
+  // records 8 q + lane / 8, field f0 + lane % 8
+  template <int f0, int AS>
+  __device__ __forceinline__ void flush() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    const int j = lane >> 3, i = lane & 7;
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      const double v = lds[8 * q + j][i];
+      if (8 * q + j < left) base[(size_t)(8 * q + j) * AS + f0 + i] = v;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  }
+};
+
 // One thread per (item, layer).  VGPR budget: the n x n matrix of the Jacobi
 // iteration (2 n^2 registers) and the factor G; two wavefronts
 // per SIMD up to n = 6, one above.
 template <int N, int S, bool MIX>
-__global__ __launch_bounds__(64, (N * S <= 6) ? 2 : 1) void k_modes(RTWork W, int M) {
+__global__ __launch_bounds__(64, (N * S <= (MIX ? 4 : 6)) ? 2 : 1) void k_modes(RTWork W, int M) {
   constexpr int n = N * S, LM = 2 * N, NT = n * (n + 1) / 2;
   constexpr bool SPLIT = n > 8;   // source terms in a second pass over the stored modes
   constexpr AOff O(N, S);
   constexpr QOff QO(N, S);
   constexpr PiOff PO(N, S);
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  const int km = W.km;
-  if (t >= W.lcnt[M]) return;   // dense (item, layer) slots of this term
+  constexpr int AS = O.size();
+  __shared__ double lds[64][9];
+  // dense (item, layer) slots of this term; lanes beyond the last repeat it
+  const int t0 = blockIdx.x * 64, nslot = W.lcnt[M], km = W.km;
+  if (t0 >= nslot) return;
+  const int t = min(t0 + (int)threadIdx.x, nslot - 1);
   const int it = W.lown[t];
   const int layer = t - W.loff[it];
+  RecordOut out{W.abuf + (size_t)t0 * AS, nslot - t0, (int)threadIdx.x, lds};
   const int NMOM = W.nmoments;
   const double* __restrict__ Qt = W.quad;
   const double* __restrict__ ph = W.phi;   // sqrt(w/mu) x the quadrature PI matrices, the table's layout
@@ -156,9 +205,6 @@ __global__ __launch_bounds__(64, (N * S <= 6) ? 2 : 1) void k_modes(RTWork W, in
   // ones belong to S for even M and to D for odd M, so for odd M the two
   // matrices, and with them E and F, change names.
   const bool odd = (M & 1) != 0;
-  double* lrec = W.abuf + il * (size_t)W.astride;
-  double* recE = lrec + (odd ? O.f(0, 0) : O.e(0, 0));
-  double* recF = lrec + (odd ? O.e(0, 0) : O.f(0, 0));
 
   double a[NT], b[NT];
   double xa[MIX ? NT : 1], xb[MIX ? NT : 1];   // antisymmetric parts (mixed)
@@ -318,10 +364,12 @@ __global__ __launch_bounds__(64, (N * S <= 6) ? 2 : 1) void k_modes(RTWork W, in
       c[k][r] = v * rdg[r];
     }
   };
-  double em[MIX ? n : 1][n];   // mixed: all of E' (the perturbation mixes the columns)
-  if constexpr (MIX) {
+  double em[SPLIT ? 1 : n][n];   // E'
+  if constexpr (!SPLIT) {
 #pragma unroll
     for (int k = 0; k < n; ++k) efcol(k, em[k]);
+  }
+  if constexpr (MIX) {
     // S' = E^T S E = K + s, D' = F^T D F = K + d with antisymmetric s, d; to
     // first order E -> E (1 + C), F -> F (1 + B) with
     //   C_jk = (k_j s_jk + k_k d_jk) / (k_k^2 - k_j^2), B_jk = (k_j d_jk + k_k s_jk) / (k_k^2 - k_j^2)
@@ -386,12 +434,38 @@ __global__ __launch_bounds__(64, (N * S <= 6) ? 2 : 1) void k_modes(RTWork W, in
       for (int r = 0; r < n; ++r) { em[k][r] += (double)de[k][r]; c[k][r] += (double)df[k][r]; }
   }
   if constexpr (SPLIT) {
-#pragma unroll
-    for (int k = 0; k < n; ++k) {
+    static_for<0, n>([&](auto kc) __attribute__((always_inline)) {
+      constexpr int k = decltype(kc)::value;
       double e[n];
       efcol(k, e);
-#pragma unroll
-      for (int r = 0; r < n; ++r) { recE[r * n + k] = e[r]; recF[r * n + k] = c[k][r]; }
+      static_for<0, n>([&](auto rc) __attribute__((always_inline)) {
+        constexpr int r = decltype(rc)::value;
+        out.put<O.e(r, k), AS>(odd ? c[k][r] : e[r]);
+      });
+      static_for<0, n>([&](auto rc) __attribute__((always_inline)) {
+        constexpr int r = decltype(rc)::value;
+        out.put<O.f(r, k), AS>(odd ? e[r] : c[k][r]);
+      });
+    });
+    // the second pass reads the lane's own record back, which other lanes
+    // wrote (a last piece that the modes leave incomplete is written again
+    // when it is full)
+    if constexpr (((2 * n * n) & 7) != 0) out.template flush<(2 * n * n) & ~7, AS>();
+    __threadfence_block();
+  } else {
+    auto rows = [&](auto first, const double (&x)[n][n]) __attribute__((always_inline)) {
+      constexpr int f0 = decltype(first)::value;
+      static_for<0, n * n>([&](auto fc) __attribute__((always_inline)) {
+        constexpr int f = decltype(fc)::value;
+        out.put<f0 + f, AS>(x[f % n][f / n]);
+      });
+    };
+    if (odd) {
+      rows(std::integral_constant<int, 0>(), c);
+      rows(std::integral_constant<int, n * n>(), em);
+    } else {
+      rows(std::integral_constant<int, 0>(), em);
+      rows(std::integral_constant<int, n * n>(), c);
     }
   }
 
@@ -478,31 +552,24 @@ __global__ __launch_bounds__(64, (N * S <= 6) ? 2 : 1) void k_modes(RTWork W, in
 
   // ---- per mode: multipliers, source coefficients, beam amplitudes
   const double sg = odd ? -1.0 : 1.0;
+  const double* lrec = W.abuf + (size_t)t * AS;
+  double otr[n], ogu[n], ogd[n], ocl[S][n], ocm[S][n];
   double spar[S];
 #pragma unroll
   for (int o = 0; o < S; ++o) spar[o] = 0.0;
   const double itw = -itrans * tdmubar;
 #pragma unroll
   for (int k = 0; k < n; ++k) {
-    double e[n];
-    if constexpr (MIX) {
-#pragma unroll
-      for (int r = 0; r < n; ++r) e[r] = em[k][r];
-    } else if constexpr (SPLIT) {
-#pragma unroll
-      for (int r = 0; r < n; ++r) e[r] = recE[r * n + k];
-    } else {
-      efcol(k, e);
-    }
-    double f[n];
+    double e[n], f[n];
 #pragma unroll
     for (int r = 0; r < n; ++r) {
-      if constexpr (SPLIT) f[r] = recF[r * n + k];
-      else f[r] = c[k][r];
-    }
-    if constexpr (!SPLIT) {
-#pragma unroll
-      for (int r = 0; r < n; ++r) { recE[r * n + k] = e[r]; recF[r * n + k] = f[r]; }
+      if constexpr (SPLIT) {
+        e[r] = lrec[(odd ? O.f(0, 0) : O.e(0, 0)) + O.e(r, k)];
+        f[r] = lrec[(odd ? O.e(0, 0) : O.f(0, 0)) + O.e(r, k)];
+      } else {
+        e[r] = em[k][r];
+        f[r] = c[k][r];
+      }
     }
     double ua[S], ub[S], qe = 0.0, qf = 0.0;
 #pragma unroll
@@ -528,8 +595,8 @@ __global__ __launch_bounds__(64, (N * S <= 6) ? 2 : 1) void k_modes(RTWork W, in
     for (int o = 0; o < S; ++o) {
       const double upup = ua[o] + ub[o], updn = sg * (ua[o] - ub[o]);
       cm[o] = lsc ? upup * h1 : 0.0;
-      lrec[O.cl(o, k)] = lsc ? updn * h2 : 0.0;
-      lrec[O.cm(o, k)] = cm[o];
+      ocl[o][k] = lsc ? updn * h2 : 0.0;
+      ocm[o][k] = cm[o];
     }
     if (beam) {
       // Green's-function amplitudes (:2649-2932)
@@ -553,12 +620,22 @@ __global__ __launch_bounds__(64, (N * S <= 6) ? 2 : 1) void k_modes(RTWork W, in
         spar[o] += updn * sd * aterm + upup * su * bterm - cm[o] * gdn;
       }
     }
-    lrec[O.t(k)] = zdel;
-    lrec[O.gup(k)] = gup;
-    lrec[O.gdn(k)] = gdn;
+    otr[k] = zdel;
+    ogu[k] = gup;
+    ogd[k] = gdn;
   }
-#pragma unroll
-  for (int o = 0; o < S; ++o) lrec[O.csrc(o)] = spar[o];
+  // the rest of the record in field order, padded to whole pieces
+  static_for<O.t(0), AS>([&](auto fc) __attribute__((always_inline)) {
+    constexpr int f = decltype(fc)::value, q = f - O.t(0), w = q / n, k = q % n;
+    double v = 0.0;
+    if constexpr (w == 0) v = otr[k];
+    else if constexpr (w == 1) v = ogu[k];
+    else if constexpr (w == 2) v = ogd[k];
+    else if constexpr (w < 3 + S) v = ocl[w - 3][k];
+    else if constexpr (w < 3 + 2 * S) v = ocm[w - 3 - S][k];
+    else if constexpr (f - O.csrc(0) < S) v = spar[f - O.csrc(0)];
+    out.put<f, AS>(v);
+  });
 }
 
 }  // namespace

@@ -121,7 +121,7 @@ struct RTWork {
   double* lev = nullptr;           // [it][km+1][4]: tauslant, suntau, atten, FO mult(enhanced)
   double* lostrans = nullptr;      // [it][km+1]
   // symmetric path (k_modes, k_adding)
-  double* abuf = nullptr;          // [it][km][astride] layer modes (AOff)
+  double* abuf = nullptr;          // [slot][astride] layer modes (AOff)
   double* pis = nullptr;           // [it][PiOff] PI functions of the user angle and the solar cosine
   int astride = 0;
   // general path (k_layer, k_bvp)
@@ -181,23 +181,29 @@ struct LOff {
   __host__ __device__ constexpr int size() const { return (2 * n * n + 5 * n + 2 * n * S + S + 1) & ~1; }
 };
 
-// Offsets inside one abuf record (per item and layer) of the symmetric path,
-// n = N*S: the modes' sum and difference vectors E(r, k), F(r, k) in the
-// scaled streams, the layer transmittances and beam amplitudes of the modes,
-// the coefficients of the upwelling source at the user angle (of the
-// down-decaying and up-decaying amplitudes) and its beam part.
+// Offsets inside one abuf record (per (item, layer) slot of the term, slot
+// numbers as in lown) of the symmetric path, n = N*S: the modes' sum and
+// difference vectors E(r, k), F(r, k) in the scaled streams, the layer
+// transmittances and beam amplitudes of the modes, the coefficients of the
+// upwelling source at the user angle (of the down-decaying and up-decaying
+// amplitudes) and its beam part.  Up to n = 8 rows are contiguous (k_adding's
+// lanes read neighbouring columns); above, where k_modes forms one mode after
+// the other, mode k's two vectors are.  Whole 64-byte pieces, so that k_modes
+// writes no partial ones.
 struct AOff {
   int n, S;
-  __host__ __device__ constexpr AOff(int N_, int S_) : n(N_ * S_), S(S_) {}
-  __host__ __device__ constexpr int e(int r, int k) const { return r * n + k; }
-  __host__ __device__ constexpr int f(int r, int k) const { return n * n + r * n + k; }
+  bool by_mode;
+  __host__ __device__ constexpr AOff(int N_, int S_) : n(N_ * S_), S(S_), by_mode(N_ * S_ > 8) {}
+  __host__ __device__ constexpr int e(int r, int k) const { return by_mode ? 2 * k * n + r : r * n + k; }
+  __host__ __device__ constexpr int f(int r, int k) const { return by_mode ? (2 * k + 1) * n + r : n * n + r * n + k; }
+  __host__ __device__ constexpr int estep() const { return by_mode ? 2 * n : 1; }   // from mode k to k + 1
   __host__ __device__ constexpr int t(int k) const { return 2 * n * n + k; }
   __host__ __device__ constexpr int gup(int k) const { return 2 * n * n + n + k; }
   __host__ __device__ constexpr int gdn(int k) const { return 2 * n * n + 2 * n + k; }
   __host__ __device__ constexpr int cl(int o, int k) const { return 2 * n * n + 3 * n + o * n + k; }
   __host__ __device__ constexpr int cm(int o, int k) const { return 2 * n * n + 3 * n + (S + o) * n + k; }
   __host__ __device__ constexpr int csrc(int o) const { return 2 * n * n + 3 * n + 2 * S * n + o; }
-  __host__ __device__ constexpr int size() const { return (2 * n * n + 3 * n + 2 * S * n + S + 1) & ~1; }
+  __host__ __device__ constexpr int size() const { return (2 * n * n + 3 * n + 2 * S * n + S + 7) & ~7; }
 };
 
 // Offsets inside one item's PI record: functions p (P; P, R, T with three
