@@ -30,24 +30,106 @@
 // Bound: the dependent chain of the 2n pivots (broadcast, reciprocal, row
 // update) per layer for small batches, the records' bytes (832 per layer at
 // N = 6) for large ones.  Measured against the pivoted band solve (k_bvp, 8 or
-// 32 lanes per item): N = 6, 400,000 items 204 -> 57 ms; one item 358 -> 51 us
-// per term; N = 12, 1,200 items 15.5 -> 2.6 ms; three Stokes components N = 4,
-// 16,000 items 133 -> 10 ms.
+// 32 lanes per item): N = 6, 400,000 items 204 -> 49 ms (2.5 TB/s of records);
+// one item 4.3 ms over its terms -> 0.13 ms (all terms side by side); N = 12,
+// 1,200 items 15.5 -> 1.3 ms; three Stokes components N = 4, 16,000 items 133 ->
+// 6.3 ms.
 #pragma once
 #include <type_traits>
 #include "rt_work.h"
 #include "rt_device.h"
 #include "rt_modes.h"
+#include "rt_converge.h"
 
 namespace aa {
 
 namespace {
 
+// Lane broadcasts.  row_newbcast reads one lane of the caller's 16-lane row in
+// all its lanes and is the one lane move that FP64 arithmetic takes as an
+// operand modifier, so a broadcast multiply-add is a single v_fmac_f64 where
+// the compiler emits a move and an FMA (k_adding, 400,000 items at N = 6 55 ->
+// 47 ms; three Stokes components N = 4, 16,000 items 9.5 -> 6.8 ms).  A DPP operand must not be read
+// within two wait states of its VALU write, and the compiler does not look
+// into asm blocks: every block starts with s_nop 1, and inside a block no
+// operand that was written before is read as a DPP operand.  All lanes of the
+// row must be active (a broadcast under a lane's own condition reads nothing).
+
 // x of lane K of the caller's 16-lane row, in all its lanes
 template <int K>
 __device__ __forceinline__ double bc16(double x) {
-  return __builtin_amdgcn_update_dpp(x, x, 0x150 + K, 0xF, 0xF, true);
+  double r;
+  asm("s_nop 1\n\tv_mov_b64_dpp %0, %1 row_newbcast:%c2 row_mask:0xf bank_mask:0xf" : "=v"(r) : "v"(x), "n"(K));
+  return r;
 }
+#define AA_DPP " row_newbcast:%c"
+#define AA_MASK " row_mask:0xf bank_mask:0xf\n\t"
+// z += a(lane I) * q and, in runs, z[j] += a(lane I + j) * q
+template <int I>
+__device__ __forceinline__ void fmac_bc(double& z, double a, double q) {
+  asm("s_nop 1\n\tv_fmac_f64_dpp %0, %1, %2" AA_DPP "3" AA_MASK : "+&v"(z) : "v"(a), "v"(q), "n"(I));
+}
+template <int I>
+__device__ __forceinline__ void fmac_bc2(double& z0, double& z1, double a, double q) {
+  asm("s_nop 1\n\tv_fmac_f64_dpp %0, %2, %3" AA_DPP "4" AA_MASK "v_fmac_f64_dpp %1, %2, %3" AA_DPP "5" AA_MASK
+      : "+&v"(z0), "+&v"(z1) : "v"(a), "v"(q), "n"(I), "n"(I + 1));
+}
+template <int I>
+__device__ __forceinline__ void fmac_bc4(double& z0, double& z1, double& z2, double& z3, double a, double q) {
+  asm("s_nop 1\n\tv_fmac_f64_dpp %0, %4, %5" AA_DPP "6" AA_MASK "v_fmac_f64_dpp %1, %4, %5" AA_DPP "7" AA_MASK
+      "v_fmac_f64_dpp %2, %4, %5" AA_DPP "8" AA_MASK "v_fmac_f64_dpp %3, %4, %5" AA_DPP "9" AA_MASK
+      : "+&v"(z0), "+&v"(z1), "+&v"(z2), "+&v"(z3)
+      : "v"(a), "v"(q), "n"(I), "n"(I + 1), "n"(I + 2), "n"(I + 3));
+}
+// z[i] += a(lane i) * q for I <= i < n
+template <int n, int I>
+__device__ __forceinline__ void fmac_run(double (&z)[n], double a, double q) {
+  if constexpr (n - I >= 4) {
+    fmac_bc4<I>(z[I], z[I + 1], z[I + 2], z[I + 3], a, q);
+    fmac_run<n, I + 4>(z, a, q);
+  } else if constexpr (n - I >= 2) {
+    fmac_bc2<I>(z[I], z[I + 1], a, q);
+    fmac_run<n, I + 2>(z, a, q);
+  } else if constexpr (n - I == 1) {
+    fmac_bc<I>(z[I], a, q);
+  }
+}
+// x[i] -= f[i](lane K) * xk for I <= i < E
+template <int n, int K, int I, int E>
+__device__ __forceinline__ void fnma_run(double (&x)[n], const double (&f)[n], double xk) {
+  if constexpr (E - I >= 4) {
+    asm("s_nop 1\n\tv_fmac_f64_dpp %0, -%4, %8" AA_DPP "9" AA_MASK "v_fmac_f64_dpp %1, -%5, %8" AA_DPP "9" AA_MASK
+        "v_fmac_f64_dpp %2, -%6, %8" AA_DPP "9" AA_MASK "v_fmac_f64_dpp %3, -%7, %8" AA_DPP "9" AA_MASK
+        : "+&v"(x[I]), "+&v"(x[I + 1]), "+&v"(x[I + 2]), "+&v"(x[I + 3])
+        : "v"(f[I]), "v"(f[I + 1]), "v"(f[I + 2]), "v"(f[I + 3]), "v"(xk), "n"(K));
+    fnma_run<n, K, I + 4, E>(x, f, xk);
+  } else if constexpr (E - I >= 2) {
+    asm("s_nop 1\n\tv_fmac_f64_dpp %0, -%2, %4" AA_DPP "5" AA_MASK "v_fmac_f64_dpp %1, -%3, %4" AA_DPP "5" AA_MASK
+        : "+&v"(x[I]), "+&v"(x[I + 1]) : "v"(f[I]), "v"(f[I + 1]), "v"(xk), "n"(K));
+    fnma_run<n, K, I + 2, E>(x, f, xk);
+  } else if constexpr (E - I == 1) {
+    asm("s_nop 1\n\tv_fmac_f64_dpp %0, -%1, %2" AA_DPP "3" AA_MASK : "+&v"(x[I]) : "v"(f[I]), "v"(xk), "n"(K));
+  }
+}
+// the same with f = x: x[i] -= x[i](lane K) * xk
+template <int n, int K, int I>
+__device__ __forceinline__ void fnma_self(double (&x)[n], double xk) {
+  if constexpr (n - I >= 4) {
+    asm("s_nop 1\n\tv_fmac_f64_dpp %0, -%0, %4" AA_DPP "5" AA_MASK "v_fmac_f64_dpp %1, -%1, %4" AA_DPP "5" AA_MASK
+        "v_fmac_f64_dpp %2, -%2, %4" AA_DPP "5" AA_MASK "v_fmac_f64_dpp %3, -%3, %4" AA_DPP "5" AA_MASK
+        : "+&v"(x[I]), "+&v"(x[I + 1]), "+&v"(x[I + 2]), "+&v"(x[I + 3]) : "v"(xk), "n"(K));
+    fnma_self<n, K, I + 4>(x, xk);
+  } else if constexpr (n - I >= 2) {
+    asm("s_nop 1\n\tv_fmac_f64_dpp %0, -%0, %2" AA_DPP "3" AA_MASK "v_fmac_f64_dpp %1, -%1, %2" AA_DPP "3" AA_MASK
+        : "+&v"(x[I]), "+&v"(x[I + 1]) : "v"(xk), "n"(K));
+    fnma_self<n, K, I + 2>(x, xk);
+  } else if constexpr (n - I == 1) {
+    asm("s_nop 1\n\tv_fmac_f64_dpp %0, -%0, %1" AA_DPP "2" AA_MASK : "+&v"(x[I]) : "v"(xk), "n"(K));
+  }
+}
+#undef AA_DPP
+#undef AA_MASK
+
 // Solves K X = X in place (lane c: column c of K and of the right-hand sides),
 // Gaussian elimination without row exchanges.  `low` collects the smallest
 // pivot.
@@ -61,46 +143,37 @@ __device__ __forceinline__ void solve16(double (&K)[n], double (&X)[n], double& 
     const double rp = rcp_nr(p);
     K[k] *= rp;
     X[k] *= rp;
-#pragma unroll
-    for (int i = k + 1; i < n; ++i) {
-      const double f = bc16<k>(K[i]);
-      X[i] = fma(-f, X[k], X[i]);
-      K[i] = fma(-f, K[k], K[i]);
-    }
+    fnma_run<n, k, k + 1, n>(X, K, X[k]);
+    fnma_self<n, k, k + 1>(K, K[k]);
   });
   static_for<0, n - 1>([&](auto kc) __attribute__((always_inline)) {
     constexpr int k = n - 1 - decltype(kc)::value;
-#pragma unroll
-    for (int i = 0; i < k; ++i) X[i] = fma(-bc16<k>(K[i]), X[k], X[i]);
+    fnma_run<n, k, 0, k>(X, K, X[k]);
   });
 }
 
 // Z = A^T Q over lanes: Z_i = sum_m A(m, i) Q_m (lane c: columns of A and Q)
 template <int n>
 __device__ __forceinline__ void mul_at(const double (&A)[n], const double (&Q)[n], double (&Z)[n]) {
-  static_for<0, n>([&](auto ic) __attribute__((always_inline)) {
-    constexpr int i = decltype(ic)::value;
-    double v = 0.0;
 #pragma unroll
-    for (int m = 0; m < n; ++m) v = fma(bc16<i>(A[m]), Q[m], v);
-    Z[i] = v;
-  });
+  for (int i = 0; i < n; ++i) Z[i] = 0.0;
+#pragma unroll
+  for (int m = 0; m < n; ++m) fmac_run<n, 0>(Z, A[m], Q[m]);
 }
-// X += sign * A Q (A given by its columns: A(i, m) is register i of lane m)
+// X -= A Q (A given by its columns: A(i, m) is register i of lane m)
 template <int n>
 __device__ __forceinline__ void sub_mul(const double (&A)[n], const double (&Q)[n], double (&X)[n]) {
   static_for<0, n>([&](auto mc) __attribute__((always_inline)) {
     constexpr int m = decltype(mc)::value;
-#pragma unroll
-    for (int i = 0; i < n; ++i) X[i] = fma(-bc16<m>(A[i]), Q[m], X[i]);
+    fnma_run<n, m, 0, n>(X, A, Q[m]);
   });
 }
 
 template <int N, int S, bool MIX>
-__global__ __launch_bounds__(64) void k_adding(RTWork W, int M, const int* __restrict__ active,
-                                               const int* __restrict__ nactive, int* __restrict__ next,
-                                               int* __restrict__ nnext) {
+__global__ __launch_bounds__(64) void k_adding(RTWork W, int M0, const int* __restrict__ active,
+                                               const int* __restrict__ nactive) {
   constexpr int n = N * S, IPW = 4;
+  const int tg = blockIdx.y, M = M0 + tg;   // this term of the group
   static_assert(n <= 15, "a lane per column and one for the vectors");
   constexpr AOff O(N, S);
   constexpr QOff QO(N, S);
@@ -135,7 +208,8 @@ __global__ __launch_bounds__(64) void k_adding(RTWork W, int M, const int* __res
 #pragma unroll
   for (int q = 0; q < IPW; ++q) Lmax = max(Lmax, __builtin_amdgcn_readlane(L, q * 16));
   const int AS = W.astride;
-  const double* __restrict__ ab = W.abuf + (size_t)W.loff[it] * AS;   // the item's slots of this term
+  // the item's slots of this term
+  const double* __restrict__ ab = W.abuf + ((size_t)tg * W.cap * km + W.loff[it]) * AS;
   const double* __restrict__ trr = W.tr + (size_t)it * km * TR_NFIELDS;
   const double* __restrict__ Qt = W.quad;
   const double ff = W.flux ? W.flux[(size_t)obs * W.nch + ch] : 1.0;
@@ -244,42 +318,64 @@ __global__ __launch_bounds__(64) void k_adding(RTWork W, int M, const int* __res
     }
   }
 
-  for (int k = Lmax - 1; k >= 0; --k) {
-    const bool here = k < L;
-    if (!here) continue;   // uniform within the item's lanes
+  // What a layer's step needs besides the modes, and the modes of the layers
+  // above, are loaded a step ahead of their use (the modes two steps up to
+  // n = 8, where the registers allow it): at the loop's top they would expose
+  // the memory latency once per layer, 1.6 us per layer for a lone item.
+  struct Step { double tk, gup, gdn, tdu, cm[S], cl[S], csrc[S]; };
+  constexpr bool AHEAD2 = n <= 8;
+  const int cl_ = col ? t : 0;
+  auto load_step = [&](int k, Step& q) __attribute__((always_inline)) {
     const double* __restrict__ lr = ab + (size_t)k * AS;
-    const int cl = col ? t : 0;
-    const double tk = col ? lr[O.t(0) + cl] : 1.0;
-    const double gup = lr[O.gup(0) + cl], gdn = lr[O.gdn(0) + cl];
-    const double tdu = trr[(size_t)k * TR_NFIELDS + TR_TDUSER];
-    // the layer above (the top: free space, E = F = 1)
-    double E1[n], F1[n];
-    if (k > 0) load_modes(k - 1, E1, F1);
-    else {
+    q.tk = lr[O.t(0) + cl_];
+    q.gup = lr[O.gup(0) + cl_];
+    q.gdn = lr[O.gdn(0) + cl_];
+    q.tdu = trr[(size_t)k * TR_NFIELDS + TR_TDUSER];
+#pragma unroll
+    for (int o = 0; o < S; ++o) {
+      q.cm[o] = lr[O.cm(o, 0) + cl_];
+      q.cl[o] = lr[O.cl(o, 0) + cl_];
+      q.csrc[o] = lr[O.csrc(o)];
+    }
+  };
+  Step cur, nxt;
+  load_step(L - 1, cur);
+  double E1[n], F1[n];   // the layer above; the top has free space (E = F = 1) above
+  double E2[AHEAD2 ? n : 1], F2[AHEAD2 ? n : 1];
+  if constexpr (AHEAD2) load_modes(L > 1 ? L - 2 : 0, E1, F1);
+
+  for (int k = Lmax - 1; k >= 0; --k) {
+    if (k >= L) continue;   // uniform within the item's lanes
+    if constexpr (AHEAD2) load_modes(k > 1 ? k - 2 : 0, E2, F2);
+    else load_modes(k > 0 ? k - 1 : 0, E1, F1);
+    load_step(k > 0 ? k - 1 : 0, nxt);
+    if (k == 0) {
 #pragma unroll
       for (int m = 0; m < n; ++m) { E1[m] = (m == t) ? 1.0 : 0.0; F1[m] = E1[m]; }
     }
+    const double tk = col ? cur.tk : 1.0, gup = cur.gup, gdn = cur.gdn, tdu = cur.tdu;
     double K[n], X[n];
     // ---- solve 1: H and H (2 gdn + z)
     static_for<0, n>([&](auto ic) __attribute__((always_inline)) {
       constexpr int i = decltype(ic)::value;
       const double one = (t == i) ? 1.0 : 0.0;
       K[i] = Z[i] + one;
-      X[i] = fma(bc16<i>(gdn), 2.0 * dvec, vec ? Z[i] : one);
+      X[i] = vec ? Z[i] : one;
+      fmac_bc<i>(X[i], gdn, 2.0 * dvec);
     });
     solve16<n>(K, X, low);
     double gg[S];
 #pragma unroll
     for (int o = 0; o < S; ++o) {
-      const double cmv = lr[O.cm(o, 0) + cl];
+      const double cmv = cur.cm[o];
       const double tv = fma(tdu, rr[o], cmv);
       double w = 0.0;
       static_for<0, n>([&](auto ic) __attribute__((always_inline)) {
         constexpr int i = decltype(ic)::value;
-        w = fma(bc16<i>(tv), X[i], w);
+        fmac_bc<i>(w, tv, X[i]);
       });
-      hh[o] = fma(tdu, hh[o], bc16<n>(w) + lr[O.csrc(o)]);
-      gg[o] = fma(tk, fma(2.0, w, -cmv), lr[O.cl(o, 0) + cl]);
+      hh[o] = fma(tdu, hh[o], bc16<n>(w) + cur.csrc[o]);
+      gg[o] = fma(tk, fma(2.0, w, -cmv), cur.cl[o]);
     }
     // ---- reflection at the layer's top and solve 2
     double A[n];
@@ -287,9 +383,12 @@ __global__ __launch_bounds__(64) void k_adding(RTWork W, int M, const int* __res
       constexpr int i = decltype(ic)::value;
       const double one = (t == i) ? 1.0 : 0.0;
       double v = vec ? X[i] : fma(2.0, X[i], -one);
-      v = fma(bc16<i>(gdn), -dvec, v);
-      v = v * tk * bc16<i>(tk);
-      v = fma(bc16<i>(gup), dvec, v);
+      fmac_bc<i>(v, gdn, -dvec);
+      v = v * tk;
+      double w = 0.0;   // (the vector's lane adds gup; every lane of the row stays active)
+      fmac_bc<i>(w, gup, dvec);
+      fmac_bc<i>(w, tk, v);
+      v = w;
       K[i] = v + one;
       X[i] = v;
     });
@@ -312,7 +411,7 @@ __global__ __launch_bounds__(64) void k_adding(RTWork W, int M, const int* __res
       double w = 0.0;
       static_for<0, n>([&](auto ic) __attribute__((always_inline)) {
         constexpr int i = decltype(ic)::value;
-        w = fma(bc16<i>(gg[o]), X[i], w);
+        fmac_bc<i>(w, gg[o], X[i]);
       });
       hh[o] -= bc16<n>(w);
       rr[o] = col ? w : 0.0;
@@ -333,7 +432,11 @@ __global__ __launch_bounds__(64) void k_adding(RTWork W, int M, const int* __res
       }
     }
 #pragma unroll
-    for (int r = 0; r < n; ++r) { E[r] = E1[r]; F[r] = F1[r]; }
+    for (int r = 0; r < n; ++r) {
+      E[r] = E1[r]; F[r] = F1[r];
+      if constexpr (AHEAD2) { E1[r] = E2[r]; F1[r] = F2[r]; }
+    }
+    cur = nxt;
   }
   // ---- no downwelling field at the top: (1 + Z) u = z, I = r . u + h
   double cum[S];
@@ -347,26 +450,74 @@ __global__ __launch_bounds__(64) void k_adding(RTWork W, int M, const int* __res
       double w = 0.0;
       static_for<0, n>([&](auto ic) __attribute__((always_inline)) {
         constexpr int i = decltype(ic)::value;
-        w = fma(bc16<i>(rr[o]), X[i], w);
+        fmac_bc<i>(w, rr[o], X[i]);
       });
       cum[o] = bc16<n>(w) + hh[o];
     }
   }
 
-  // ---- Fourier convergence on the item's lane 0, or hand-over to k_rescue
-  bool goes_on = false;
   if (t == 0 && valid) {
-    if (W.nfour[it] != 0 || !(low > 1.0e-9)) {
-      W.nfour[it] = M + 1;   // (k_rescue takes the item up at this term)
-      W.rlist[atomicAdd(W.rcnt, 1)] = it;
-    } else {
-      goes_on = converge_term<N, S>(W, it, obs, oi, ff, M, cum);
+    const size_t e = (size_t)it * W.terms + tg;
+#pragma unroll
+    for (int o = 0; o < S; ++o) W.cums[e * S + o] = cum[o];
+    if (!(low > 1.0e-9)) W.tflag[e] = 1;
+  }
+}
+
+// The convergence test over a group's terms in order, one lane per item: an
+// item that is done has its outputs written, one with a marked term goes to
+// k_rescue at that term, the others enter the next group's lists.
+template <int N, int S>
+__global__ __launch_bounds__(64) void k_converge(RTWork W, int M0, int terms, const int* __restrict__ active,
+                                                 const int* __restrict__ nactive, int* __restrict__ next,
+                                                 int* __restrict__ nnext, int* __restrict__ lnext) {
+  const int lane = threadIdx.x;
+  int first = -1, cntb = 0;
+  const int* lst = active;
+  {
+    int acc = 0;
+#pragma unroll
+    for (int b = 0; b < LBINS; ++b) {
+      const int c = nactive[b], nbk = (c + 63) / 64;
+      if (first < 0 && (int)blockIdx.x < acc + nbk) {
+        first = ((int)blockIdx.x - acc) * 64;
+        cntb = c;
+        lst = active + (size_t)b * W.cap;
+      }
+      acc += nbk;
     }
   }
-  const int noff = append_items(W, it, L, goes_on, nnext, next, W.lcnt + M + 1);
-  const int goff = __builtin_amdgcn_ds_bpermute(4 * (lane - t), noff);
-  if (goff >= 0)
-    for (int l = t; l < L; l += 16) W.lown[goff + l] = it;
+  if (first < 0) return;   // uniform over the wavefront
+  const bool valid = first + lane < cntb;
+  const int it = lst[valid ? first + lane : first];
+  const int L = W.L_it[it];
+  bool goes_on = false;
+  if (valid) {
+    const int gi = global_item(W, it), obs = gi / W.nch, ch = gi - obs * W.nch;
+    const size_t oi = (size_t)ch * W.nobs + obs;
+    const double ff = W.flux ? W.flux[(size_t)obs * W.nch + ch] : 1.0;
+    for (int g = 0; g < terms; ++g) {
+      const size_t e = (size_t)it * W.terms + g;
+      if (W.tflag[e] != 0) {
+        W.nfour[it] = M0 + g + 1;
+        W.rlist[atomicAdd(W.rcnt, 1)] = it;
+        goes_on = false;
+        break;
+      }
+      double cum[S];
+#pragma unroll
+      for (int o = 0; o < S; ++o) cum[o] = W.cums[e * S + o];
+      goes_on = converge_term<N, S>(W, it, obs, oi, ff, M0 + g, cum);
+      if (!goes_on) break;
+    }
+  }
+  const int off = append_items(W, it, L, goes_on, nnext, next, lnext);
+  // the wavefront fills the slots of one item after the other
+  for (unsigned long long todo = __ballot(off >= 0); todo != 0ull; todo &= todo - 1ull) {
+    const int j = __ffsll((long long)todo) - 1;
+    const int oj = __shfl(off, j, 64), Lj = __shfl(L, j, 64), ij = __shfl(it, j, 64);
+    for (int l = lane; l < Lj; l += 64) W.lown[oj + l] = ij;
+  }
 }
 
 }  // namespace

@@ -1129,7 +1129,8 @@ typedef double d4v __attribute__((ext_vector_type(4)));
 // the accumulator rows of lane l are 4*(l/16) + v for f32 but l/16 + 4*v for
 // f64 (v = 0..3; checked on the device with a probe of known products).
 template <int N, int S, typename T, int PG>
-__global__ __launch_bounds__(64) void k_sabdab(RTWork W, int M) {
+__global__ __launch_bounds__(64) void k_sabdab(RTWork W, int M0, int group) {
+  const int tg = blockIdx.y, M = M0 + tg;   // this term of the group (the general path's groups are one term)
   constexpr bool F64 = std::is_same<T, double>::value;
   using V4 = typename std::conditional<F64, d4v, f4v>::type;
   constexpr int n = N * S, LM = 2 * N;
@@ -1140,10 +1141,10 @@ __global__ __launch_bounds__(64) void k_sabdab(RTWork W, int M) {
   constexpr bool PRE = sab_tiles(N, S) <= 32;   // A tiles held in registers
   const int lane = threadIdx.x;
   const int km = W.km;
-  const int nl = W.lcnt[M];
+  const int nl = W.lcnt[group];
   const int kq = lane >> 4;
   bool valid[SAB_PG];
-  size_t il[SAB_PG];
+  size_t il[SAB_PG], ol[SAB_PG];
   bool any = false;
 #pragma unroll
   for (int q = 0; q < SAB_PG; ++q) {
@@ -1154,6 +1155,7 @@ __global__ __launch_bounds__(64) void k_sabdab(RTWork W, int M) {
     const int layer = v ? (int)(p - W.loff[it]) : 0;
     valid[q] = v;
     il[q] = (size_t)it * km + layer;
+    ol[q] = (size_t)tg * W.cap * km + il[q];
     any = any || v;
   }
   if (__ballot(any) == 0ull) return;
@@ -1184,8 +1186,8 @@ __global__ __launch_bounds__(64) void k_sabdab(RTWork W, int M) {
 #pragma unroll
   for (int q = 0; q < SAB_PG; ++q) {
   T* out;
-  if constexpr (F64) out = W.sab64 + il[q] * (size_t)ROWS;
-  else out = W.sab32 + il[q] * (size_t)ROWS;
+  if constexpr (F64) out = W.sab64 + ol[q] * (size_t)ROWS;
+  else out = W.sab32 + ol[q] * (size_t)ROWS;
 #pragma unroll
   for (int rt = 0; rt < RT; ++rt) {
     V4 c = {(T)0, (T)0, (T)0, (T)0};
@@ -1267,32 +1269,39 @@ __global__ __launch_bounds__(64) void k_rescue(RTWork W) {
   }
 }
 
-// The Fourier terms of a chunk on the symmetric path.
+// The Fourier terms of a chunk on the symmetric path, W.terms of them at a
+// time.  The slot count of group j is lcnt[j].
 template <int N, int S, bool MIX, int PG>
 int fourier_loop_sym(const RTWork& W, int nitems, int* const lists[2], int* counts, hipStream_t st) {
   const int nl = (int)(((size_t)nitems * W.km + 63) / 64);
   const int ns = (int)(((size_t)nitems * W.km + 16 * PG - 1) / (16 * PG));
-  const int nb = (nitems + 3) / 4 + LBINS;
+  const int nb = (nitems + 3) / 4 + LBINS, nc = (nitems + 63) / 64 + LBINS;
   prof_begin(PROF_ITEM, st);
   hipLaunchKernelGGL((k_pi<N, S>), dim3((unsigned)(((size_t)nitems * 2 * N + 63) / 64)), dim3(64), 0, st, W, nitems);
   prof_end(PROF_ITEM, st);
-  for (int M = 0; M <= W.nmoments; ++M) {
-    const int* in = lists[M & 1];
-    int* out = lists[(M + 1) & 1];
+  bool mid = W.mid_event != nullptr;
+  for (int M = 0, j = 0; M <= W.nmoments; M += W.terms, ++j) {
+    const int* in = lists[j & 1];
+    int* out = lists[(j + 1) & 1];
+    const unsigned ng = (unsigned)std::min(W.terms, W.nmoments - M + 1);
     if constexpr (needs_sabdab(N, S, MIX)) {
       prof_begin(PROF_SABDAB, st);
-      hipLaunchKernelGGL((k_sabdab<N, S, typename std::conditional<MIX, float, double>::type, PG>), dim3(ns), dim3(64),
-                         0, st, W, M);
+      hipLaunchKernelGGL((k_sabdab<N, S, typename std::conditional<MIX, float, double>::type, PG>), dim3(ns, ng),
+                         dim3(64), 0, st, W, M, j);
       prof_end(PROF_SABDAB, st);
     }
     prof_begin(PROF_LAYER, st);
-    hipLaunchKernelGGL((k_modes<N, S, MIX>), dim3(nl), dim3(64), 0, st, W, M);
+    hipLaunchKernelGGL((k_modes<N, S, MIX>), dim3(nl, ng), dim3(64), 0, st, W, M, j);
     prof_end(PROF_LAYER, st);
     prof_begin(PROF_BVP, st);
-    hipLaunchKernelGGL((k_adding<N, S, MIX>), dim3(nb), dim3(64), 0, st, W, M, in, counts + M * LBINS, out,
-                       counts + (M + 1) * LBINS);
+    hipLaunchKernelGGL((k_adding<N, S, MIX>), dim3(nb, ng), dim3(64), 0, st, W, M, in, counts + j * LBINS);
+    hipLaunchKernelGGL((k_converge<N, S>), dim3(nc), dim3(64), 0, st, W, M, (int)ng, in, counts + j * LBINS, out,
+                       counts + (j + 1) * LBINS, W.lcnt + j + 1);
     prof_end(PROF_BVP, st);
-    if (W.mid_event && M == std::min(W.mid_term, W.nmoments)) AA_CHECK(hipEventRecord(W.mid_event, st));
+    if (mid && M + (int)ng > std::min(W.mid_term, W.nmoments)) {
+      AA_CHECK(hipEventRecord(W.mid_event, st));
+      mid = false;
+    }
   }
   prof_begin(PROF_BVP, st);
   hipLaunchKernelGGL((k_rescue<N, S, MIX>), dim3(W.rblocks), dim3(64), 0, st, W);
@@ -1313,7 +1322,7 @@ int fourier_loop_shape(const RTWork& W, int nitems, int* const lists[2], int* co
     int* out = lists[(M + 1) & 1];
     prof_begin(PROF_SABDAB, st);
     hipLaunchKernelGGL((k_sabdab<N, S, typename std::conditional<MIX, float, double>::type, PG>), dim3(ns), dim3(64), 0,
-                       st, W, M);
+                       st, W, M, M);
     prof_end(PROF_SABDAB, st);
     prof_begin(PROF_LAYER, st);
     hipLaunchKernelGGL((k_layer<N, S, MIX>), dim3(nl), dim3(64), 0, st, W, M);

@@ -33,7 +33,7 @@
 //
 // An item with a layer whose S or D is not positive definite, whose Jacobi
 // iteration does not converge, or whose eigenmatrix is partially isolated
-// (some rows without off-diagonal elements) is marked in W.nfour and continues
+// (some rows without off-diagonal elements) is marked in W.tflag and continues
 // on the reference's general eigensolver and banded solve (k_rescue).
 //
 // Mixed precision: SAB/DAB come from the FP32 contraction and are symmetric
@@ -180,7 +180,7 @@ struct RecordOut {
 // iteration (2 n^2 registers) and the factor G; two wavefronts
 // per SIMD up to n = 6, one above.
 template <int N, int S, bool MIX>
-__global__ __launch_bounds__(64, (N * S <= (MIX ? 4 : 6)) ? 2 : 1) void k_modes(RTWork W, int M) {
+__global__ __launch_bounds__(64, (N * S <= (MIX ? 4 : 6)) ? 2 : 1) void k_modes(RTWork W, int M0, int group) {
   constexpr int n = N * S, LM = 2 * N, NT = n * (n + 1) / 2;
   constexpr bool SPLIT = n > 8;   // source terms in a second pass over the stored modes
   constexpr AOff O(N, S);
@@ -189,12 +189,14 @@ __global__ __launch_bounds__(64, (N * S <= (MIX ? 4 : 6)) ? 2 : 1) void k_modes(
   constexpr int AS = O.size();
   __shared__ double lds[64][9];
   // dense (item, layer) slots of this term; lanes beyond the last repeat it
-  const int t0 = blockIdx.x * 64, nslot = W.lcnt[M], km = W.km;
+  const int t0 = blockIdx.x * 64, nslot = W.lcnt[group], km = W.km;
   if (t0 >= nslot) return;
   const int t = min(t0 + (int)threadIdx.x, nslot - 1);
   const int it = W.lown[t];
   const int layer = t - W.loff[it];
-  RecordOut out{W.abuf + (size_t)t0 * AS, nslot - t0, (int)threadIdx.x, lds};
+  const int tg = blockIdx.y, M = M0 + tg;   // this term of the group
+  const size_t sb = (size_t)tg * W.cap * km;
+  RecordOut out{W.abuf + (sb + t0) * AS, nslot - t0, (int)threadIdx.x, lds};
   const int NMOM = W.nmoments;
   const double* __restrict__ Qt = W.quad;
   const double* __restrict__ ph = W.phi;   // sqrt(w/mu) x the quadrature PI matrices, the table's layout
@@ -234,8 +236,8 @@ __global__ __launch_bounds__(64, (N * S <= (MIX ? 4 : 6)) ? 2 : 1) void k_modes(
   } else {
     using TSD = typename std::conditional<MIX, float, double>::type;
     const TSD* rec;
-    if constexpr (MIX) rec = W.sab32 + il * (size_t)(2 * n * n);
-    else rec = W.sab64 + il * (size_t)(2 * n * n);
+    if constexpr (MIX) rec = W.sab32 + (sb + il) * (size_t)(2 * n * n);
+    else rec = W.sab64 + (sb + il) * (size_t)(2 * n * n);
     const TSD* ra = rec + (odd ? n * n : 0);
     const TSD* rb = rec + (odd ? 0 : n * n);
 #pragma unroll
@@ -332,7 +334,7 @@ __global__ __launch_bounds__(64, (N * S <= (MIX ? 4 : 6)) ? 2 : 1) void k_modes(
     }
     ok = ok && conv;
   }
-  if (!ok) W.nfour[it] = 1;
+  if (!ok) W.tflag[(size_t)it * W.terms + tg] = 1;
 
   // c = k v: E' = G v / sqrt(k), then F' = sqrt(k) G^-T v in place of c
   double keig[n], rsk[n];   // k, 1 / sqrt(k)
@@ -552,7 +554,7 @@ __global__ __launch_bounds__(64, (N * S <= (MIX ? 4 : 6)) ? 2 : 1) void k_modes(
 
   // ---- per mode: multipliers, source coefficients, beam amplitudes
   const double sg = odd ? -1.0 : 1.0;
-  const double* lrec = W.abuf + (size_t)t * AS;
+  const double* lrec = W.abuf + (sb + t) * AS;
   double otr[n], ogu[n], ogd[n], ocl[S][n], ocm[S][n];
   double spar[S];
 #pragma unroll

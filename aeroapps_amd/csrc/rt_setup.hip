@@ -816,6 +816,8 @@ __global__ void k_item(RTWork W, int nitems, int* active, int* nactive) {
 __global__ __launch_bounds__(64) void k_enlist(RTWork W, int nitems, int* active, int* nactive) {
   const int it = blockIdx.x * 64 + threadIdx.x;
   const bool take = it < nitems && W.status[it] == 0;
+  if (take && W.tflag)
+    for (int g = 0; g < W.terms; ++g) W.tflag[(size_t)it * W.terms + g] = 0;
   append_items(W, it, take ? W.L_it[it] : 0, take, nactive, active, W.lcnt);
 }
 

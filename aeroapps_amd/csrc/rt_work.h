@@ -121,7 +121,11 @@ struct RTWork {
   double* lev = nullptr;           // [it][km+1][4]: tauslant, suntau, atten, FO mult(enhanced)
   double* lostrans = nullptr;      // [it][km+1]
   // symmetric path (k_modes, k_adding)
-  double* abuf = nullptr;          // [slot][astride] layer modes (AOff)
+  // (terms: Fourier terms of a group, whose kernels run in one launch each)
+  int terms = 1;
+  double* abuf = nullptr;          // [term of the group][slot][astride] layer modes (AOff)
+  double* cums = nullptr;          // [it][terms][S] Fourier components of the TOA Stokes vector
+  int* tflag = nullptr;            // [it][terms] 1: the term is for k_rescue
   double* pis = nullptr;           // [it][PiOff] PI functions of the user angle and the solar cosine
   int astride = 0;
   // general path (k_layer, k_bvp)
@@ -225,6 +229,23 @@ constexpr int SYM_MAX_N = 12, SYM_MAX_N_MIXED = 7;
 __host__ __device__ constexpr bool sym_path(int N, int S, bool mixed) {
   return N * S <= (mixed ? SYM_MAX_N_MIXED : SYM_MAX_N);
 }
+// Fourier terms per group on the symmetric path.  The terms of an item do not
+// depend on each other until the convergence test, so a small batch runs
+// several side by side (down to one launch for all of them) instead of one
+// after the other; k_converge drops what an item turns out not to need.  A
+// lone item leaves the GPU empty and takes 12 terms in the time of one (k_adding
+// 620 -> 121 us at N = 6).  From TERM_PAIRS (item, term) pairs on k_modes, one
+// thread per layer, is throughput-bound and a speculative term costs what it
+// takes (1,200 items at N = 12: groups of 13 made k_modes 2.8 -> 5.0 ms), while
+// k_adding, 4 pairs per wavefront, still gains from two terms up to about twice
+// as many items; the largest batches go term by term.
+constexpr int TERM_PAIRS = 4096;
+inline int term_group(int nitems, int nmoments) {
+  int g = nitems > 0 ? TERM_PAIRS / nitems : 1;
+  if (g < 2) g = nitems <= 2 * TERM_PAIRS ? 2 : 1;
+  return g > nmoments + 1 ? nmoments + 1 : g;
+}
+
 // SAB/DAB from k_sabdab: always in the mixed path, with three Stokes
 // components, and on the general path (the symmetric scalar FP64 path forms
 // the two triangles in k_modes).

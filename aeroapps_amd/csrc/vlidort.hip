@@ -347,7 +347,9 @@ size_t carve_work(Carver& C, RTWork& W, int cap) {
   const bool sym = sym_path(W.N, W.S, mixed);
   W.astride = AOff(W.N, W.S).size();
   if (sym) {
-    W.abuf = C.take<double>((size_t)cap * km * W.astride);
+    W.abuf = C.take<double>((size_t)cap * km * W.astride * W.terms);
+    W.cums = C.take<double>((size_t)cap * W.terms * W.S);
+    W.tflag = C.take<int>((size_t)cap * W.terms);
     W.pis = C.take<double>((size_t)cap * PiOff(W.N, W.S).size());
     W.rlist = C.take<int>(cap);
     // workgroups of k_rescue: up to 512, fewer for small chunks, so that their
@@ -360,8 +362,9 @@ size_t carve_work(Carver& C, RTWork& W, int cap) {
   }
   W.brdf = (W.kernel_wt || W.u10m || W.bpdf) ? C.take<double>((size_t)cap * W.brdf_stride) : nullptr;
   W.wsa_cache = W.kernel_wt ? C.take<double>(4) : nullptr;
-  W.sab32 = mixed ? C.take<float>((size_t)cap * km * 2 * n * n) : nullptr;
-  W.sab64 = (!mixed && needs_sabdab(W.N, W.S, mixed)) ? C.take<double>((size_t)cap * km * 2 * n * n) : nullptr;
+  const size_t sabs = (size_t)cap * km * 2 * n * n * (sym ? W.terms : 1);
+  W.sab32 = mixed ? C.take<float>(sabs) : nullptr;
+  W.sab64 = (!mixed && needs_sabdab(W.N, W.S, mixed)) ? C.take<double>(sabs) : nullptr;
   return C.off;
 }
 
@@ -433,12 +436,19 @@ int run_items(RTWork W, int g0, int g1, hipStream_t st, const int* d_items = nul
                            std::max<size_t>(1, btab.size()) * sizeof(double) +
                            sizeof(int) * ((LBINS + 1) * (W.nmoments + 2) + 1) +
                            rescue_doubles(W.N, W.S, W.km) * sizeof(double) + 16 * 256;
-  if (fixed_base) {
-    const size_t per = bytes_per_item(W) + 2 * LBINS * sizeof(int);
-    if (fixed_bytes <= tab_bytes + per) return AA_EDIMS;
-    capi = (fixed_bytes - tab_bytes) / per;
-  } else if (work_cap_items(W, &capi)) {
-    return AA_EHIP;
+  // Fourier terms per group: as many as the batch's size calls for, one where
+  // a group's records would not leave the batch in one chunk
+  W.terms = term_group(nitems, W.nmoments);
+  for (;;) {
+    if (fixed_base) {
+      const size_t per = bytes_per_item(W) + 2 * LBINS * sizeof(int);
+      if (fixed_bytes <= tab_bytes + per && W.terms == 1) return AA_EDIMS;
+      capi = fixed_bytes <= tab_bytes + per ? 0 : (fixed_bytes - tab_bytes) / per;
+    } else if (work_cap_items(W, &capi)) {
+      return AA_EHIP;
+    }
+    if (W.terms == 1 || capi >= (size_t)nitems) break;
+    W.terms = 1;
   }
   // chunks of equal size: a small remainder chunk would run every Fourier
   // term on a nearly idle GPU
