@@ -13,6 +13,42 @@ namespace aa {
 // Fortran SIGN(a,b)
 __device__ __forceinline__ double fsign(double a, double b) { return b >= 0.0 ? fabs(a) : -fabs(a); }
 
+#if defined(__HIP_DEVICE_COMPILE__)
+// 1/x and 1/sqrt(x) of normal positive or negative x: the hardware
+// approximation and Newton steps (about 1 ulp), without the scaling and
+// special-case code of the library division and square root.
+__device__ __forceinline__ double rcp_nr(double x) {
+  double y = __builtin_amdgcn_rcp(x);
+  y = fma(y, fma(-x, y, 1.0), y);
+  return fma(y, fma(-x, y, 1.0), y);
+}
+__device__ __forceinline__ double rsqrt_nr(double x) {
+  double y = __builtin_amdgcn_rsq(x);
+  double h = 0.5 * y;
+  double e = fma(-x * y, h, 0.5);
+  y = fma(y, e, y);
+  h = 0.5 * y;
+  e = fma(-x * y, h, 0.5);
+  return fma(y, e, y);
+}
+// sqrt(x), x > 0, from the same start (Goldschmidt steps and a correction)
+__device__ __forceinline__ double sqrt_nr(double x) {
+  const double y = __builtin_amdgcn_rsq(x);
+  double g = x * y, h = 0.5 * y;
+  double r = fma(-h, g, 0.5);
+  g = fma(g, r, g);
+  h = fma(h, r, h);
+  r = fma(-h, g, 0.5);
+  g = fma(g, r, g);
+  h = fma(h, r, h);
+  return fma(fma(-g, g, x), h, g);
+}
+#else
+__device__ double rcp_nr(double);
+__device__ double rsqrt_nr(double);
+__device__ double sqrt_nr(double);
+#endif
+
 // Taylor_series_1 (REG/vlidort_Taylor.f90:119-133)
 __device__ __forceinline__ double taylor1(double eps, double delta, double udel, double sm) {
   double d[TAYLOR_ORDER + 2];

@@ -56,24 +56,6 @@ namespace aa {
 
 namespace {
 
-// 1/x and 1/sqrt(x) of normal positive or negative x: the hardware
-// approximation and Newton steps (about 1 ulp), without the scaling and
-// special-case code of the library division and square root.
-__device__ __forceinline__ double rcp_nr(double x) {
-  double y = __builtin_amdgcn_rcp(x);
-  y = fma(y, fma(-x, y, 1.0), y);
-  return fma(y, fma(-x, y, 1.0), y);
-}
-__device__ __forceinline__ double rsqrt_nr(double x) {
-  double y = __builtin_amdgcn_rsq(x);
-  double h = 0.5 * y;
-  double e = fma(-x * y, h, 0.5);
-  y = fma(y, e, y);
-  h = 0.5 * y;
-  e = fma(-x * y, h, 0.5);
-  return fma(y, e, y);
-}
-
 // compile-time loop: f(integral_constant<int, B>) .. f(integral_constant<int, E - 1>)
 template <int B, int E, class F>
 __device__ __forceinline__ void static_for(F&& f) {
