@@ -18,6 +18,7 @@
 #include "prof.h"
 
 #include <algorithm>
+#include <type_traits>
 #include <cctype>
 #include <cmath>
 #include <cstring>
@@ -71,7 +72,19 @@ constexpr int MAXTR = 32;
 //     is a 256-byte coalesced load from L2; the KC layers give KC independent
 //     accumulations per tracer.  Per output element the order is the
 //     reference's (tracer order; (pm*ssa_i)*tau_i).
+//
+// V4 (moments, table rows and bases in whole groups of four, 32-bit element
+// offsets): step 3 has a lane per four moments of one layer, so W lanes cover a
+// layer's moments and 64 / W layers run side by side.  A row read is then one
+// 16-byte load per lane instead of four 4-byte loads of four lanes' worth of
+// address arithmetic and LDS broadcasts, which bounded the kernel (20 VALU
+// instructions per (layer, tracer, moment) where the arithmetic is 7): 400,000
+// (column, channel) pairs x 64 moments 28.8 -> 16.5 ms, 50,003 x 32 6.4 -> 1.5,
+// 16,000 x six sets of 32 4.7 -> 1.6, one pair 51 -> 22 us.  Each output element
+// sees the same operations in the same order.
 constexpr int MIE_KC_MAX = 8, MIE_CAP = 128;   // layers per chunk, (layer, tracer) slots
+constexpr int mie_w4(int nmom) { return nmom <= 32 ? 8 : (nmom <= 64 ? 16 : (nmom <= 128 ? 32 : 64)); }
+template <int W4>   // lanes per layer in step 3; 0: lane = moment
 __global__ void __launch_bounds__(64) get_aop_kernel(MieDev T, int km, int nobs, int nch, int nq,
                                                      const int* __restrict__ tracer_idx,
                                                      const int* __restrict__ chan_idx,
@@ -108,7 +121,11 @@ __global__ void __launch_bounds__(64) get_aop_kernel(MieDev T, int km, int nobs,
           const float g_in = lin(T.g[tb + s.irh], T.g[tb + s.irhp1], s.arh);
           const float q = qm[((long)i * nq + iq) * km + k];
           info[e] = make_float4(__int_as_float(s.irh), s.arh, __fdiv_rn(bsca_in, bext_in), __fmul_rn(bext_in, q));
-          rows[e] = make_int4((int)tb + s.irh, (int)tb + s.irhp1, (npol == 6 && T.npol_t[tr] == 4) ? 1 : 0, 1);
+          const int tied = (npol == 6 && T.npol_t[tr] == 4) ? 1 : 0;
+          if constexpr (W4 > 0)   // element offsets of the rows
+            rows[e] = make_int4((int)((tb + s.irh) * rowstride), (int)((tb + s.irhp1) * rowstride), tied, 1);
+          else
+            rows[e] = make_int4((int)tb + s.irh, (int)tb + s.irhp1, tied, 1);
           gin[e] = g_in;
         } else {
           rows[e] = make_int4(0, 0, 0, 0);
@@ -141,7 +158,92 @@ __global__ void __launch_bounds__(64) get_aop_kernel(MieDev T, int km, int nobs,
     __syncthreads();
     // ---- 3. lane = moment.  Polarisations run in pairs (a, b) where the
     //      spherical extension ties b to a's running sum (P22 = P11, P44 = P33).
-    if (pmom_o != nullptr) {
+    if constexpr (W4 > 0) {
+      constexpr int G = 64 / W4 < MIE_KC_MAX ? 64 / W4 : MIE_KC_MAX, R = MIE_KC_MAX / G;
+      const int grp = lane / W4;   // this lane's layers: grp R .. grp R + R - 1
+      for (int m0 = 0; m0 < nmom; m0 += 4 * W4) {
+        const int m = m0 + 4 * (lane - grp * W4);
+        const bool mon = m < nmom && grp < G;
+        const int mr = m < nmom ? m : 0;
+        for (int ps = 0; ps < npass; ++ps) {
+          int pa = ps, pb = -1;
+          if (npol == 6) {
+            pa = (ps == 0) ? 0 : (ps == 1) ? 2 : (ps == 2) ? 1 : 3;
+            pb = (ps == 0) ? 4 : (ps == 1) ? 5 : -1;
+          }
+          const float* ta = T.pmom + pa * T.nmom + mr;
+          const float* tbp = T.pmom + (pb >= 0 ? pb : 0) * T.nmom + mr;
+          float acc_a[R][4], acc_b[R][4];
+#pragma unroll
+          for (int r = 0; r < R; ++r)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) { acc_a[r][q] = 0.0f; acc_b[r][q] = 0.0f; }
+          for (int iq = 0; iq < ntr_eff; ++iq) {
+            // tracer found and tied polarisations: the same for every layer
+            const int4 r0 = rows[iq];
+            if (r0.w == 0) continue;
+            const bool sph = r0.z != 0;
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+              const int kk = min(grp * R + r, kc - 1);
+              const float4 inf = info[kk * ntr + iq];
+              const int4 rr = rows[kk * ntr + iq];
+              const float4 lo = *reinterpret_cast<const float4*>(ta + (unsigned)rr.x);
+              const float4 hi = *reinterpret_cast<const float4*>(ta + (unsigned)rr.y);
+              const float l4[4] = {lo.x, lo.y, lo.z, lo.w}, h4[4] = {hi.x, hi.y, hi.z, hi.w};
+#pragma unroll
+              for (int q = 0; q < 4; ++q)
+                acc_a[r][q] = __fadd_rn(acc_a[r][q], __fmul_rn(__fmul_rn(lin(l4[q], h4[q], inf.y), inf.z), inf.w));
+              if (pb >= 0) {
+                if (sph) {
+#pragma unroll
+                  for (int q = 0; q < 4; ++q) acc_b[r][q] = acc_a[r][q];
+                } else {
+                  const float4 lb = *reinterpret_cast<const float4*>(tbp + (unsigned)rr.x);
+                  const float4 hb = *reinterpret_cast<const float4*>(tbp + (unsigned)rr.y);
+                  const float lb4[4] = {lb.x, lb.y, lb.z, lb.w}, hb4[4] = {hb.x, hb.y, hb.z, hb.w};
+#pragma unroll
+                  for (int q = 0; q < 4; ++q)
+                    acc_b[r][q] =
+                        __fadd_rn(acc_b[r][q], __fmul_rn(__fmul_rn(lin(lb4[q], hb4[q], inf.y), inf.z), inf.w));
+                }
+              }
+            }
+          }
+          if (mon) {
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+              const float st = stl[min(grp * R + r, kc - 1)];
+              if (normalize && st > 0.0f) {
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                  acc_a[r][q] = __fdiv_rn(acc_a[r][q], st);
+                  if (pb >= 0) acc_b[r][q] = __fdiv_rn(acc_b[r][q], st);
+                }
+              }
+            }
+            // a moment's layers are contiguous: the lanes of the groups store
+            // its 8 layers side by side
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+              float* oa = pmom_o + ((long)pa * nmom + m + q) * ostride + obase + k0 + grp * R;
+              float* ob = pb >= 0 ? pmom_o + ((long)pb * nmom + m + q) * ostride + obase + k0 + grp * R : nullptr;
+              if (R == 2 && kc == MIE_KC_MAX && (((size_t)oa | (size_t)ob) & 7) == 0) {
+                *reinterpret_cast<float2*>(oa) = make_float2(acc_a[0][q], acc_a[R - 1][q]);
+                if (ob) *reinterpret_cast<float2*>(ob) = make_float2(acc_b[0][q], acc_b[R - 1][q]);
+              } else {
+#pragma unroll
+                for (int r = 0; r < R; ++r)
+                  if (grp * R + r < kc) {
+                    oa[r] = acc_a[r][q];
+                    if (ob) ob[r] = acc_b[r][q];
+                  }
+              }
+            }
+          }
+        }
+      }
+    } else if (pmom_o != nullptr) {
       for (int m0 = 0; m0 < nmom; m0 += 64) {
         const int m = m0 + lane;
         const bool mon = m < nmom;
@@ -387,9 +489,22 @@ int launch_get_aop(const aa_mie* t, int km, int nobs, int nch, int nq, const int
   const int kc = std::max(1, std::min(MIE_KC_MAX, MIE_CAP / std::max(1, ntr_eff)));
   const int ny = blocks <= 32768 ? (km + kc - 1) / kc : 1;
   prof_begin(PROF_MIE, st);
-  hipLaunchKernelGGL(get_aop_kernel, dim3((unsigned)blocks, (unsigned)ny), dim3(64), 0, st, t->dev, km, nobs, nch, nq,
-                     d_tracer_idx, d_chan_idx, d_qm, d_rh, nmom, npol, ntr_eff, normalize, d_tau, d_ssa, d_g,
-                     d_pmom);
+  const dim3 grid((unsigned)blocks, (unsigned)ny);
+  auto launch = [&](auto w4) {
+    hipLaunchKernelGGL((get_aop_kernel<decltype(w4)::value>), grid, dim3(64), 0, st, t->dev, km, nobs, nch, nq,
+                       d_tracer_idx, d_chan_idx, d_qm, d_rh, nmom, npol, ntr_eff, normalize, d_tau, d_ssa, d_g,
+                       d_pmom);
+  };
+  // four moments per lane where rows, moments and the table base come in whole
+  // aligned groups of four and element offsets fit 32 bits
+  const long elems = (long)t->dev.ntracer * t->dev.nch * t->dev.nrh * t->dev.npol * t->dev.nmom;
+  const bool v4 = d_pmom && nmom % 4 == 0 && t->dev.nmom % 4 == 0 && ((size_t)t->dev.pmom & 15) == 0 &&
+                  elems <= 0x7fffffffL;
+  if (!v4) launch(std::integral_constant<int, 0>());
+  else if (mie_w4(nmom) == 8) launch(std::integral_constant<int, 8>());
+  else if (mie_w4(nmom) == 16) launch(std::integral_constant<int, 16>());
+  else if (mie_w4(nmom) == 32) launch(std::integral_constant<int, 32>());
+  else launch(std::integral_constant<int, 64>());
   prof_end(PROF_MIE, st);
   AA_CHECK(hipGetLastError());
   return 0;
