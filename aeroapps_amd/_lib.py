@@ -43,6 +43,8 @@ SIGNATURES = {
     "aa_get_aop_vector_dev": (_ci, [_vp, _ci, _ci, _ci, _ci, _vp, _vp, _vp, _vp, _ci, _ci, _vp, _vp, _vp, _vp, _vp]),
     "aa_vlidort_scalar_lambert": (_ci, [_ci, _ci, _ci, _dp, _ci, _ci, _ci, _ci, _dp, _dp, _dp, _dp, _dp, _dp, _dp,
                                         _dp, _dp, _dp, _dp, _dp, _dp, _cd, _ci, _ci, _dp, _dp, _ip, _ip]),
+    "aa_vlidort_scalar_lambert_f32": (_ci, [_ci, _ci, _ci, _ci, _ci, _ci, _ci, _dp, _dp, _fp, _fp, _fp, _dp, _dp, _dp,
+                                            _dp, _dp, _cd, _ci, _dp, _dp, _ip, _ip]),
     "aa_vlidort_vector_lambert": (_ci, [_ci, _ci, _ci, _dp, _ci, _ci, _ci, _ci, _dp, _dp, _dp, _dp, _dp, _dp, _dp,
                                         _dp, _dp, _dp, _dp, _dp, _dp, _dp, _cd, _ci, _ci, _dp, _dp, _dp, _dp, _ip,
                                         _ip]),

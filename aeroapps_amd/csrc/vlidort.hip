@@ -524,6 +524,12 @@ int host_call_block(size_t bytes, char** out) { return arena_reserve(nullptr, AR
 
 namespace {
 
+// Layer optics in float32 (as the Chem_Mie calls return them) instead of
+// lambert_host's double arguments: widened exactly, on the device.
+struct HostOptics32 {
+  const float *tau, *ssa, *pmom;
+};
+
 int lambert_host(bool vector, int km, int nch, int nobs, int nstreams, int plane_parallel, int nmom, int npol,
                  const double* rot, const double* depol, const double* alpha, const double* tau, const double* ssa,
                  const double* pmom, const double* he, const double* albedo, const double* sza, const double* raa,
@@ -532,7 +538,7 @@ int lambert_host(bool vector, int km, int nch, int nobs, int nstreams, int plane
                  const double* kernel_wt = nullptr, const double* kparam = nullptr, double* br = nullptr,
                  const double* u10m = nullptr, const double* v10m = nullptr, const double* mr = nullptr,
                  bool stokes1 = false, const int* host_latch = nullptr, const double* bpdf = nullptr,
-                 double* br_q = nullptr, double* br_u = nullptr) {
+                 double* br_q = nullptr, double* br_u = nullptr, const HostOptics32* o32 = nullptr) {
   if (!rc) return AA_EARG;
   *rc = 0;
   const bool cx = u10m != nullptr;
@@ -542,8 +548,8 @@ int lambert_host(bool vector, int km, int nch, int nobs, int nstreams, int plane
   const bool modis = kernel_wt != nullptr || cx;   // a BRDF surface instead of the albedo
   const bool surf_brdf = modis || pol;             // the radiance runs on a BRDF record
   if (km <= 0 || nch <= 0 || nobs < 0 || nmom <= 0 || npol <= 0) return AA_EARG;
-  if (!rot || !depol || !tau || !ssa || !pmom || !he || (!albedo && !modis) || !sza || !raa || !vza || !radiance ||
-      !reflectance)
+  if (!rot || !depol || (!o32 && (!tau || !ssa || !pmom)) || (o32 && (!o32->tau || !o32->ssa || !o32->pmom)) || !he ||
+      (!albedo && !modis) || !sza || !raa || !vza || !radiance || !reflectance)
     return AA_EARG;
   if (kernel_wt && ((vector && !pol) || !kparam || !br)) return AA_EARG;
   // VLIDORT_Init of the BRDF drivers (V283/VLIDORT_Mod.F90:369) rejects nMom
@@ -578,9 +584,10 @@ int lambert_host(bool vector, int km, int nch, int nobs, int nstreams, int plane
     d.rot = C.take<double>(nl);
     d.depol = C.take<double>(nch);
     d.alpha = (vector && alpha) ? C.take<double>(nl) : nullptr;
-    d.tau = C.take<double>(nl);
-    d.ssa = C.take<double>(nl);
-    d.pmom = C.take<double>(nl * nmom * npol);
+    const size_t ow = o32 ? 2 : 1;   // floats in half the doubles' space
+    d.tau = C.take<double>((nl + ow - 1) / ow);
+    d.ssa = C.take<double>((nl + ow - 1) / ow);
+    d.pmom = C.take<double>((nl * nmom * npol + ow - 1) / ow);
     d.he = C.take<double>((size_t)(km + 1) * nobs);
     d.albedo = modis ? nullptr : C.take<double>(no);
     d.kw = kernel_wt ? C.take<double>(no * 3) : nullptr;
@@ -613,8 +620,13 @@ int lambert_host(bool vector, int km, int nch, int nobs, int nstreams, int plane
   auto up = [](double* dst, const double* src, size_t n) {
     return (n && src) ? hipMemcpy(dst, src, n * sizeof(double), hipMemcpyHostToDevice) : hipSuccess;
   };
-  if (up(d.rot, rot, nl) || up(d.depol, depol, nch) || (d.alpha && up(d.alpha, alpha, nl)) || up(d.tau, tau, nl) ||
-      up(d.ssa, ssa, nl) || up(d.pmom, pmom, nl * nmom * npol) || up(d.he, he, (size_t)(km + 1) * nobs) ||
+  auto up32 = [](double* dst, const float* src, size_t n) {
+    return n ? hipMemcpy(dst, src, n * sizeof(float), hipMemcpyHostToDevice) : hipSuccess;
+  };
+  if (o32 ? (up32(d.tau, o32->tau, nl) || up32(d.ssa, o32->ssa, nl) || up32(d.pmom, o32->pmom, nl * nmom * npol))
+          : (up(d.tau, tau, nl) || up(d.ssa, ssa, nl) || up(d.pmom, pmom, nl * nmom * npol)))
+    return AA_EHIP;
+  if (up(d.rot, rot, nl) || up(d.depol, depol, nch) || (d.alpha && up(d.alpha, alpha, nl)) || up(d.he, he, (size_t)(km + 1) * nobs) ||
       (d.albedo && up(d.albedo, albedo, no)) || (d.kw && up(d.kw, kernel_wt, no * 3)) ||
       (d.kp && up(d.kp, kparam, no * 2)) || (d.u10 && up(d.u10, u10m, nobs)) || (d.v10 && up(d.v10, v10m, nobs)) ||
       (d.mr && up(d.mr, mr, nch)) || up(d.sza, sza, nobs) || up(d.raa, raa, nobs) || up(d.vza, vza, nobs) ||
@@ -622,7 +634,7 @@ int lambert_host(bool vector, int km, int nch, int nobs, int nstreams, int plane
     return AA_EHIP;
   W.rot = d.rot; W.depol = d.depol; W.alpha = d.alpha;
   W.tau = d.tau; W.ssa = d.ssa; W.pmom = d.pmom;
-  W.optics_f32 = 0; W.opt_obs0 = 0; W.opt_nobs = nobs;
+  W.optics_f32 = o32 ? 1 : 0; W.opt_obs0 = 0; W.opt_nobs = nobs;
   W.he = d.he; W.albedo = d.albedo;
   W.kernel_wt = d.kw; W.kparam = d.kp;
   W.u10m = d.u10; W.v10m = d.v10; W.mr = d.mr;
@@ -780,6 +792,19 @@ int aa_vlidort_scalar_lambert(int km, int nch, int nobs, const double* channels,
   return aa::lambert_host(false, km, nch, nobs, nstreams, plane_parallel, nmom, npol, rot, depol, nullptr, tau, ssa,
                           pmom, he, albedo, solar_zenith, relat_azymuth, sensor_zenith, nullptr, missing, precision,
                           radiance, reflectance, nullptr, nullptr, nfourier, rc);
+}
+
+int aa_vlidort_scalar_lambert_f32(int km, int nch, int nobs, int nstreams, int plane_parallel, int nmom, int npol,
+                                  const double* rot, const double* depol, const float* tau, const float* ssa,
+                                  const float* pmom, const double* he, const double* albedo,
+                                  const double* solar_zenith, const double* relat_azymuth,
+                                  const double* sensor_zenith, double missing, int precision, double* radiance,
+                                  double* reflectance, int* nfourier, int* rc) {
+  const aa::HostOptics32 o{tau, ssa, pmom};
+  return aa::lambert_host(false, km, nch, nobs, nstreams, plane_parallel, nmom, npol, rot, depol, nullptr, nullptr,
+                          nullptr, nullptr, he, albedo, solar_zenith, relat_azymuth, sensor_zenith, nullptr, missing,
+                          precision, radiance, reflectance, nullptr, nullptr, nfourier, rc, nullptr, nullptr, nullptr,
+                          nullptr, nullptr, nullptr, false, nullptr, nullptr, nullptr, nullptr, &o);
 }
 
 int aa_vlidort_vector_lambert(int km, int nch, int nobs, const double* channels, int nstreams, int plane_parallel,

@@ -14,7 +14,7 @@ import ctypes
 
 import numpy as np
 
-from ._lib import check, lib, _dp, _ip
+from ._lib import check, lib, _dp, _fp, _ip
 
 
 def _f64(a):
@@ -25,10 +25,39 @@ def _ptr(a, kind=_dp):
     return a.ctypes.data_as(kind)
 
 
+def _all_f32(*arrs):
+    return all(isinstance(a, np.ndarray) and a.dtype == np.float32 and a.flags.f_contiguous for a in arrs)
+
+
+def _scalar_lambert_f32(nstreams, plane_parallel, ROT, depol, tau, ssa, pmom, he, albedo, sza, raa, vza, MISSING,
+                        precision, return_nfourier):
+    ROT, depol, he, albedo, sza, raa, vza = map(_f64, (ROT, depol, he, albedo, sza, raa, vza))
+    km, nch, nobs = tau.shape
+    nmom, npol = pmom.shape[3], pmom.shape[4] if pmom.ndim == 5 else 1
+    rad = np.zeros((nobs, nch), order="F")
+    refl = np.zeros((nobs, nch), order="F")
+    nf = np.zeros((nobs, nch), dtype=np.int32, order="F")
+    rc = np.zeros(1, dtype=np.int32)
+    e = lib().aa_vlidort_scalar_lambert_f32(km, nch, nobs, int(nstreams), int(bool(plane_parallel)), nmom, npol,
+                                            _ptr(ROT), _ptr(depol), _ptr(tau, _fp), _ptr(ssa, _fp), _ptr(pmom, _fp),
+                                            _ptr(he), _ptr(albedo), _ptr(sza), _ptr(raa), _ptr(vza), float(MISSING),
+                                            int(precision), _ptr(rad), _ptr(refl), _ptr(nf, _ip), _ptr(rc, _ip))
+    check(e, "aa_vlidort_scalar_lambert")
+    if return_nfourier:
+        return rad, refl, int(rc[0]), nf
+    return rad, refl, int(rc[0])
+
+
 def scalar_lambert(channels, nstreams, plane_parallel, ROT, depol, tau, ssa, g, pmom, pe, he, te, albedo,
                    solar_zenith, relat_azymuth, sensor_zenith, MISSING, verbose=0, precision=0,
                    return_nfourier=False):
-    """VLIDORT_Scalar_Lambert (src/Components/rtms/geo_vlidort/VLIDORT_LAMBERT.F90:34-168)."""
+    """VLIDORT_Scalar_Lambert (src/Components/rtms/geo_vlidort/VLIDORT_LAMBERT.F90:34-168).
+
+    Layer optics that are float32 in Fortran order, as get_aop_vector returns
+    them, go to the device as they are and are widened there."""
+    if _all_f32(tau, ssa, pmom) and tau.ndim == 3 and ssa.shape == tau.shape and pmom.shape[:3] == tau.shape:
+        return _scalar_lambert_f32(nstreams, plane_parallel, ROT, depol, tau, ssa, pmom, he, albedo, solar_zenith,
+                                   relat_azymuth, sensor_zenith, MISSING, precision, return_nfourier)
     channels, ROT, depol, tau, ssa, g, pmom, pe, he, te, albedo, sza, raa, vza = map(
         _f64, (channels, ROT, depol, tau, ssa, g, pmom, pe, he, te, albedo, solar_zenith, relat_azymuth,
                sensor_zenith))

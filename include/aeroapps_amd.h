@@ -205,6 +205,18 @@ int aa_vlidort_scalar_lambert(int km, int nch, int nobs, const double* channels,
                               const double* sensor_zenith, double missing, int verbose, int precision,
                               double* radiance, double* reflectance, int* nfourier, int* rc);
 
+/* No counterpart in the reference: aa_vlidort_scalar_lambert with the layer
+ * optics in float32, as aa_get_aop_vector returns them (half the bytes over
+ * PCIe, widened exactly on the device; the same results), and without the
+ * arguments that the driver does not read. */
+int aa_vlidort_scalar_lambert_f32(int km, int nch, int nobs, int nstreams, int plane_parallel, int nmom, int npol,
+                                  const double* rot, const double* depol, const float* tau, const float* ssa,
+                                  const float* pmom, const double* he, const double* albedo,
+                                  const double* solar_zenith, const double* relat_azymuth,
+                                  const double* sensor_zenith, double missing, int precision, double* radiance,
+                                  double* reflectance, int* nfourier, int* rc);
+
+
 int aa_vlidort_vector_lambert(int km, int nch, int nobs, const double* channels, int nstreams,
                               int plane_parallel, int nmom, int npol, const double* rot, const double* depol,
                               const double* alpha, const double* tau, const double* ssa, const double* pmom,

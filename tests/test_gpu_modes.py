@@ -131,3 +131,20 @@ def test_partial_isolation_is_missing(gpu):
                                           pm.T, cols.pe.T, cols.he.T, cols.te.T, cols.albedo.T, cols.sza, cols.raa,
                                           cols.vza, cols.flux_factor.T, S.MISSING, return_nfourier=True)
     assert (I == S.MISSING).all() and (Q == S.MISSING).all() and (U == S.MISSING).all() and (nf == 0).all()
+
+
+@pytest.mark.parametrize("ncol,km,nch,nmom", [(3, 7, 1, 9), (1, 1, 1, 1), (5, 6, 2, 32)])
+@pytest.mark.parametrize("precision", [0, 1])
+def test_float32_optics_give_the_same_bits(gpu, ncol, km, nch, nmom, precision):
+    """Fortran-ordered float32 optics take their own entry point; the results
+    are those of the widened arrays, bit for bit."""
+    print(f"case float32 optics ncol={ncol} km={km} nmom={nmom}", flush=True)
+    cols = S.make_columns(ncol, km, CH[:nch], seed=29)
+    tabs = S.make_mie_tables(CH[:nch], nmom=nmom, npol=1)
+    tau, ssa, g, pm, _ = CM.get_aop_vector(tabs, CH[:nch], tabs[0].lambda_m, S.TRACERS, cols.qm, cols.rh, nmom, 1)
+    f = lambda a: np.asarray(a, dtype=np.float64)
+    wide = scalar(cols, f(tau), f(ssa), f(g), f(pm), 3, cols.albedo, precision)
+    half = scalar(cols, tau, ssa, g, pm, 3, cols.albedo, precision)
+    assert tau.dtype == np.float32
+    for a, b in zip(wide, half):
+        assert np.array_equal(a, b)
