@@ -225,7 +225,7 @@ __global__ __launch_bounds__(64) void k_adding(RTWork W, int M0, const int* __re
     const int c = col ? t : 0;
 #pragma unroll
     for (int m = 0; m < n; ++m) {
-      const double x = r[O.e(m, 0) + c * O.estep()], y = r[O.f(m, 0) + c * O.estep()];
+      const double x = r[O.e(m, c)], y = r[O.f(m, c)];
       e[m] = col ? x : 0.0;
       f[m] = col ? y : 0.0;
     }
@@ -327,14 +327,14 @@ __global__ __launch_bounds__(64) void k_adding(RTWork W, int M0, const int* __re
   const int cl_ = col ? t : 0;
   auto load_step = [&](int k, Step& q) __attribute__((always_inline)) {
     const double* __restrict__ lr = ab + (size_t)k * AS;
-    q.tk = lr[O.t(0) + cl_];
-    q.gup = lr[O.gup(0) + cl_];
-    q.gdn = lr[O.gdn(0) + cl_];
+    q.tk = lr[O.t(cl_)];
+    q.gup = lr[O.gup(cl_)];
+    q.gdn = lr[O.gdn(cl_)];
     q.tdu = trr[(size_t)k * TR_NFIELDS + TR_TDUSER];
 #pragma unroll
     for (int o = 0; o < S; ++o) {
-      q.cm[o] = lr[O.cm(o, 0) + cl_];
-      q.cl[o] = lr[O.cl(o, 0) + cl_];
+      q.cm[o] = lr[O.cm(o, cl_)];
+      q.cl[o] = lr[O.cl(o, cl_)];
       q.csrc[o] = lr[O.csrc(o)];
     }
   };

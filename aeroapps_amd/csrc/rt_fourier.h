@@ -2,7 +2,7 @@
 //
 // Two paths per (streams, Stokes, precision) class (sym_path, rt_work.h).  The
 // symmetric path (k_pi, k_modes in rt_modes.h, k_adding in rt_adding.h) solves
-// symmetric eigenproblems and adds the layers; it takes n = N*S <= 12 in FP64
+// symmetric eigenproblems and adds the layers; it takes n = N*S <= 15 in FP64
 // and n <= 7 mixed.  The general path below serves the larger classes and, item
 // by item (k_rescue), what the symmetric path hands over:
 //
@@ -1291,7 +1291,8 @@ int fourier_loop_sym(const RTWork& W, int nitems, int* const lists[2], int* coun
       prof_end(PROF_SABDAB, st);
     }
     prof_begin(PROF_LAYER, st);
-    hipLaunchKernelGGL((k_modes<N, S, MIX>), dim3(nl, ng), dim3(64), 0, st, W, M, j);
+    if constexpr (N * S > 8) hipLaunchKernelGGL((k_modes_pair<N, S>), dim3(2 * nl, ng), dim3(64), 0, st, W, M, j);
+    else hipLaunchKernelGGL((k_modes<N, S, MIX>), dim3(nl, ng), dim3(64), 0, st, W, M, j);
     prof_end(PROF_LAYER, st);
     prof_begin(PROF_BVP, st);
     hipLaunchKernelGGL((k_adding<N, S, MIX>), dim3(nb, ng), dim3(64), 0, st, W, M, in, counts + j * LBINS);

@@ -190,24 +190,30 @@ struct LOff {
 // difference vectors E(r, k), F(r, k) in the scaled streams, the layer
 // transmittances and beam amplitudes of the modes, the coefficients of the
 // upwelling source at the user angle (of the down-decaying and up-decaying
-// amplitudes) and its beam part.  Up to n = 8 rows are contiguous (k_adding's
-// lanes read neighbouring columns); above, where k_modes forms one mode after
-// the other, mode k's two vectors are.  Whole 64-byte pieces, so that k_modes
-// writes no partial ones.
+// amplitudes) and its beam part.  Up to n = 8 (k_modes) each quantity is
+// contiguous over the modes, as k_adding's lanes read it, in whole 64-byte
+// pieces; above (k_modes_pair, a lane per half of the modes) a mode's
+// quantities are, so that a lane writes one stream.
 struct AOff {
   int n, S;
   bool by_mode;
   __host__ __device__ constexpr AOff(int N_, int S_) : n(N_ * S_), S(S_), by_mode(N_ * S_ > 8) {}
-  __host__ __device__ constexpr int e(int r, int k) const { return by_mode ? 2 * k * n + r : r * n + k; }
-  __host__ __device__ constexpr int f(int r, int k) const { return by_mode ? (2 * k + 1) * n + r : n * n + r * n + k; }
-  __host__ __device__ constexpr int estep() const { return by_mode ? 2 * n : 1; }   // from mode k to k + 1
-  __host__ __device__ constexpr int t(int k) const { return 2 * n * n + k; }
-  __host__ __device__ constexpr int gup(int k) const { return 2 * n * n + n + k; }
-  __host__ __device__ constexpr int gdn(int k) const { return 2 * n * n + 2 * n + k; }
-  __host__ __device__ constexpr int cl(int o, int k) const { return 2 * n * n + 3 * n + o * n + k; }
-  __host__ __device__ constexpr int cm(int o, int k) const { return 2 * n * n + 3 * n + (S + o) * n + k; }
-  __host__ __device__ constexpr int csrc(int o) const { return 2 * n * n + 3 * n + 2 * S * n + o; }
-  __host__ __device__ constexpr int size() const { return (2 * n * n + 3 * n + 2 * S * n + S + 7) & ~7; }
+  __host__ __device__ constexpr int block() const { return 2 * n + 3 + 2 * S; }   // one mode
+  __host__ __device__ constexpr int e(int r, int k) const { return by_mode ? k * block() + r : r * n + k; }
+  __host__ __device__ constexpr int f(int r, int k) const {
+    return by_mode ? k * block() + n + r : n * n + r * n + k;
+  }
+  // per-mode scalar w (0 transmittance, 1 / 2 beam amplitudes at the top / bottom, 3.. source)
+  __host__ __device__ constexpr int w(int w_, int k) const {
+    return by_mode ? k * block() + 2 * n + w_ : 2 * n * n + w_ * n + k;
+  }
+  __host__ __device__ constexpr int t(int k) const { return w(0, k); }
+  __host__ __device__ constexpr int gup(int k) const { return w(1, k); }
+  __host__ __device__ constexpr int gdn(int k) const { return w(2, k); }
+  __host__ __device__ constexpr int cl(int o, int k) const { return w(3 + o, k); }
+  __host__ __device__ constexpr int cm(int o, int k) const { return w(3 + S + o, k); }
+  __host__ __device__ constexpr int csrc(int o) const { return n * block() + o; }
+  __host__ __device__ constexpr int size() const { return (n * block() + S + 7) & ~7; }
 };
 
 // Offsets inside one item's PI record: functions p (P; P, R, T with three
@@ -221,14 +227,15 @@ struct PiOff {
 };
 
 // Whether a (streams, Stokes, precision) class runs on the symmetric path.
-// FP64: n = N*S <= 12, where the Jacobi iteration's matrix (2 n^2 registers)
-// still fits the register file of a lane.  Mixed: n <= 7, where E and F fit
-// together (the perturbation step mixes their columns); from N = 8 on the
-// mixed path's FP32 source assembly belongs to k_layer.
-constexpr int SYM_MAX_N = 12, SYM_MAX_N_MIXED = 7;
+// FP64: n = N*S <= 15, the columns that k_adding's 16 lanes hold beside the
+// vectors.  Mixed: n <= 7, where E and F fit one lane's registers together (the
+// perturbation step mixes their columns); from N = 8 on the mixed path's FP32
+// source assembly belongs to k_layer.
+constexpr int SYM_MAX_N = 15, SYM_MAX_N_MIXED = 7;
 __host__ __device__ constexpr bool sym_path(int N, int S, bool mixed) {
   return N * S <= (mixed ? SYM_MAX_N_MIXED : SYM_MAX_N);
 }
+
 // Fourier terms per group on the symmetric path.  The terms of an item do not
 // depend on each other until the convergence test, so a small batch runs
 // several side by side (down to one launch for all of them) instead of one
@@ -246,12 +253,9 @@ inline int term_group(int nitems, int nmoments) {
   return g > nmoments + 1 ? nmoments + 1 : g;
 }
 
-// SAB/DAB from k_sabdab: always in the mixed path, with three Stokes
-// components, and on the general path (the symmetric scalar FP64 path forms
-// the two triangles in k_modes).
-__host__ __device__ constexpr bool needs_sabdab(int N, int S, bool mixed) {
-  return mixed || S != 1 || !sym_path(N, S, mixed);
-}
+// SAB/DAB from k_sabdab: in the mixed path and on the general path (in FP64 the
+// symmetric path forms its two triangles where it factorises them).
+__host__ __device__ constexpr bool needs_sabdab(int N, int S, bool mixed) { return mixed || !sym_path(N, S, mixed); }
 
 // Offsets inside one bbuf record: surface reflection terms of the bottom
 // layer for the current Fourier term, per quadrature row i < N (the

@@ -48,7 +48,7 @@ def check_scalar(cols, tau, ssa, g, pm, N, albedo, precision=0):
 @pytest.mark.parametrize("N,ncol,km,nch,precision", [
     (1, 1, 1, 1, 0), (1, 5, 72, 1, 0), (2, 3, 2, 2, 0), (2, 4, 9, 1, 1), (3, 17, 30, 1, 0), (5, 2, 72, 2, 1),
     (7, 9, 11, 1, 1), (7, 1, 72, 1, 0), (8, 5, 40, 1, 0), (8, 3, 40, 1, 1), (10, 3, 20, 1, 0), (12, 6, 72, 1, 0),
-    (12, 2, 5, 1, 1), (13, 2, 6, 1, 0)])
+    (12, 2, 5, 1, 1), (13, 2, 6, 1, 0), (9, 7, 3, 1, 0), (14, 35, 1, 1, 0), (15, 3, 24, 1, 0)])
 def test_scalar_edges(gpu, N, ncol, km, nch, precision):
     print(f"case scalar N={N} ncol={ncol} km={km} precision={precision}", flush=True)
     cols, *opt = inputs(ncol, km, nch, 32, 1, seed=71 + N)
