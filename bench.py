@@ -32,16 +32,21 @@ PEAK_FP64_TFLOPS = 78.6
 PEAK_FP32_MFMA_TFLOPS = 157.3
 PEAK_HBM_GBS = 8000.0
 PROF_NAMES = ["mie", "check", "optics", "geom", "item", "layer", "bvp", "brdf", "sabdab"]
-# HBM bytes per item-term (read, written) of the radiance kernels at N=6
-# scalar, keyed (kernel, N, S, mixed), from FETCH_SIZE/WRITE_SIZE counter runs
-# scaled by a copy-kernel calibration
-# (profiles/hbm_traffic_40k_columns_4ch_12streams.md)
-TRAFFIC_PER_ITEM_TERM = {("bvp", 6, 1, False): (153.2e3, 10.9e3), ("bvp", 6, 1, True): (153.2e3, 10.9e3),
-                         ("layer", 6, 1, False): (55.2e3, 84.1e3), ("layer", 6, 1, True): (34.6e3, 86.7e3)}
+# Bytes per item-term (read, written) of the radiance kernels at N=6 scalar and
+# 72 layers, keyed (kernel, N, S, mixed): the layer records of 90 doubles that
+# k_modes writes and k_adding reads, with the coefficients (and in the mixed
+# path the FP32 SAB/DAB block) and transmittances that they are made from
+TRAFFIC_PER_ITEM_TERM = {("bvp", 6, 1, False): (56.4e3, 0.1e3), ("bvp", 6, 1, True): (56.4e3, 0.1e3),
+                         ("layer", 6, 1, False): (11.5e3, 51.8e3), ("layer", 6, 1, True): (32.3e3, 51.8e3)}
+
+
+def symmetric(N, S_, mixed):
+    """Whether a class runs on the symmetric path (k_modes, k_adding)."""
+    return N * S_ <= (7 if mixed else 15)
 
 
 # ----------------------------------------------------------------- algorithmic work
-def flops_per_term(N, S_, L, nmoments, M):
+def flops_per_term(N, S_, L, nmoments, M, sym):
     """Algorithmic FP64 flops of one (column, channel) at Fourier term M:
     eigensystem (F_b), boundary-value solve (F_c) and source (F_d).  F_b is
     returned without its SAB/DAB contraction term 4 s n^2 Lm per layer (that
@@ -53,10 +58,17 @@ def flops_per_term(N, S_, L, nmoments, M):
     solve U^T w = c with the running w . b' (per eliminated column: w_j, its
     product with b'_j, and the update of the accumulators of the row's
     remaining columns, per Stokes output); F_d the source functional c, d
-    (per layer S (2n + 2) + 1).  An FMA counts as 2 flops."""
+    (per layer S (2n + 2) + 1).  On the symmetric path (`sym`) F_b is the two
+    triangles, their Cholesky factors, G^T L, three sweeps of column rotations
+    (8n flops each), E, F and the products with the source vectors, F_c the
+    layer adding (about 13 n^3 per layer), F_d 0.  An FMA counts as 2 flops."""
     n = S_ * N
     n2 = 2 * n
     Lm = nmoments - M + 1
+    if sym:
+        Fb = L * (n * (n + 1) * Lm * S_ + 2 * n ** 3 + 3 * (n * (n - 1) // 2) * 8 * n + 2 * n ** 3
+                  + 4 * n * n * (S_ + 1))
+        return Fb, L * 13 * n ** 3, 0
     Fb = L * (4 * N * S_ ** 3 * Lm + 2 * n ** 3 + 25 * n ** 3)
     mid = sum((3 * n - 1 - i) * (1 + 2 * (4 * n - i)) for i in range(n2))
     last = sum((2 * n - 1 - i) * (1 + 2 * (2 * n - i)) for i in range(n2))
@@ -339,7 +351,8 @@ def main():
     combos, cnts = np.unique(np.stack([n_it, l_it, nfh[ok]]), axis=1, return_counts=True)
     for (n_c, l_c, terms), cnt in zip(combos.T, cnts):
         for M in range(int(terms)):
-            b_, c_, d_ = flops_per_term(int(n_c), Sx, int(l_c), min(2 * int(n_c) - 1, nmom), M)
+            b_, c_, d_ = flops_per_term(int(n_c), Sx, int(l_c), min(2 * int(n_c) - 1, nmom), M,
+                                        symmetric(int(n_c), Sx, rmx is not None))
             fb += cnt * b_; fc += cnt * c_; fd += cnt * d_
             f_, b4_ = sabdab_per_term(int(n_c), Sx, int(l_c), min(2 * int(n_c) - 1, nmom), M, 4)
             sab_f += cnt * f_; sab_b4 += cnt * b4_
@@ -366,19 +379,21 @@ def main():
 
     def roofline(kname):
         """FP64-VALU roofline of one radiance kernel over the timed region:
-        algorithmic flops (k_layer: F_b without the SAB/DAB contraction, which
-        k_sabdab performs; k_bvp: structural F_c + F_d) over the kernel's total
-        HIP-event time; HBM traffic per launch from the counter constants."""
+        algorithmic flops (F_b for k_modes or k_layer, F_c + F_d for k_adding
+        or k_bvp) over the kernel's total HIP-event time; traffic per launch
+        from the record sizes."""
+        sym = symmetric(N or max(wl["stream_choices"]), Sx, rmx is not None)
+        shown = {"layer": "modes", "bvp": "adding"}[kname] if sym else kname
         ms = kms[kname]
         launches = max(1, kln[kname])
         flops = fb if kname == "layer" else fc + fd
         ach = flops / (ms / 1000.0) / 1e12
         r = {"bound": "fp64_valu", "achieved": round(ach, 3), "peak": PEAK_FP64_TFLOPS, "unit": "TFLOP/s",
              "frac": round(ach / PEAK_FP64_TFLOPS, 4), "traffic": None,
-             "kernel": (f"k_{kname}<{N},{Sx}>" if wl["nstreams"] is not None
-                        else f"k_{kname}<{min(wl['stream_choices'])}..{N},{Sx}>"),
+             "kernel": (f"k_{shown}<{N},{Sx}>" if wl["nstreams"] is not None
+                        else f"k_{shown}<{min(wl['stream_choices'])}..{N},{Sx}>"),
              "kernel_avg_ms": round(ms / launches, 4), "kernel_launches": int(launches),
-             "flops": ("F_b without the SAB/DAB term" if kname == "layer" else "F_c + F_d (structural)"),
+             "flops": ("F_b" if kname == "layer" else "F_c + F_d") + ("" if sym else " (structural, without SAB/DAB)"),
              "note": "FP64 vector ALU work (no MFMA); peak is the MI355X FP64 vector rate"}
         key = (kname, N, Sx, rmx is not None)
         if key in TRAFFIC_PER_ITEM_TERM and wl["nstreams"] is not None and not uneven and not modis:
