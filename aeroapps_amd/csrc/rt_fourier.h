@@ -1340,14 +1340,15 @@ int fourier_loop_shape(const RTWork& W, int nitems, int* const lists[2], int* co
 
 // The launch shapes of W.shape_bvp / W.shape_sab (0: default, 1: the
 // alternative the tuner may pick); the band solver's shapes exist on the
-// general path only.
+// general path only, k_sabdab's where it runs.
 template <int N, int S, bool MIX>
 int fourier_loop_prec(const RTWork& W, int nitems, int* const lists[2], int* counts, hipStream_t st) {
   constexpr int n = N * S;
   constexpr int P0 = sab_groups(N, S), P1 = sab_groups_alt(N, S);
   const bool gb = W.shape_bvp == 1, gs = W.shape_sab == 1;
   if constexpr (sym_path(N, S, MIX)) {
-    if (gs) return fourier_loop_sym<N, S, MIX, P1>(W, nitems, lists, counts, st);
+    if constexpr (needs_sabdab(N, S, MIX))
+      if (gs) return fourier_loop_sym<N, S, MIX, P1>(W, nitems, lists, counts, st);
     return fourier_loop_sym<N, S, MIX, P0>(W, nitems, lists, counts, st);
   } else {
     constexpr int G0 = bvp_group(n), G1 = bvp_group_alt(n);
