@@ -518,8 +518,10 @@ __device__ void geom_level(const RTWork& W, int ita, unsigned cm, int n, int nto
 
   // ---- Chapman ray (non-refractive): impact parameter and start
   const double mu_toa = cos(sza * DEG_TO_RAD), sn_toa = sqrt(1.0 - mu_toa * mu_toa);
+  // (cos(sza) below 7.5e-9 rounds sn_toa to 1 and the ray starts at its tangent
+  // point, where sqrt_nr does not hold)
   const double bch = planpar ? 0.0 : sn_toa * rn;
-  double cch = sqrt_nr((rn - bch) * (rn + bch));
+  double cch = bch < rn ? sqrt_nr((rn - bch) * (rn + bch)) : 0.0;
   double tau[CH];
 #pragma unroll
   for (int c = 0; c < CH; ++c) tau[c] = 0.0;
