@@ -773,8 +773,11 @@ __global__ __launch_bounds__(64) void k_item(RTWork W) {
         const double u = __shfl_up(v, d, 64);
         if (lane >= d) v += u;
       }
+      // (the depth above is the lane before's sum, not v - dt: that would leave
+      // the rounding of a thick layer's own depth)
+      const double above = __shfl_up(v, 1, 64);
       tl[q] = (carry + v) * sec0;
-      tp[q] = (carry + (v - dt[q])) * sec0;
+      tp[q] = (lane == 0 ? carry : carry + above) * sec0;
       carry += __shfl(v, 63, 64);
     } else {
       tl[q] = on ? lev[(size_t)nl * 4] : 0.0;

@@ -48,3 +48,16 @@ def test_sun_at_the_horizon(gpu, sza):
     assert np.max(np.abs(I[ok] / I0[ok] - 1.0)) < 3.0e-4
     assert np.max(np.abs(R[ok] / R0[ok] - 1.0)) < 3.0e-4
     assert (nf[ok] == nf0[ok]).all()
+
+
+@pytest.mark.parametrize("thick", [0, 20, 62, 63, 64, 71])
+def test_plane_parallel_depth_above_a_thick_layer(gpu, thick):
+    """The beam at the top of a layer is that of the layers above it, however
+    thick the layer itself is: a difference of inclusive sums would leave
+    1e10 x 1.1e-16 = 1e-6 in the slant depth."""
+    print(f"case plane-parallel thick layer {thick}", flush=True)
+    cols, tau, ssa, g, pm = inputs(7, 72, seed=11)
+    tau[:, :, thick] = 1.0e10
+    I, R, nf, I0, R0, nf0 = both(cols, tau, ssa, g, pm, 4, True)
+    assert max_rel(I, I0) < RTOL_FP64 and max_rel(R, R0) < RTOL_FP64
+    assert (nf == nf0).all()
