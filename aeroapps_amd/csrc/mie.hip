@@ -487,7 +487,8 @@ int launch_get_aop(const aa_mie* t, int km, int nobs, int nch, int nq, const int
   // the GPU anyhow and a wavefront walks its column's chunks (400,000 pairs:
   // 28.5 ms, apart 30.1).
   const int kc = std::max(1, std::min(MIE_KC_MAX, MIE_CAP / std::max(1, ntr_eff)));
-  const int ny = blocks <= 32768 ? (km + kc - 1) / kc : 1;
+  // (a grid's second dimension ends at 65,536; a wavefront then walks several)
+  const int ny = blocks <= 32768 ? std::min((km + kc - 1) / kc, 65536) : 1;
   prof_begin(PROF_MIE, st);
   const dim3 grid((unsigned)blocks, (unsigned)ny);
   auto launch = [&](auto w4) {
