@@ -110,7 +110,8 @@ __device__ __forceinline__ double dpp_d(double x) {
 // Layer solution of one (item, layer) at Fourier term M on the general path:
 // SAB/DAB in srec, the layer record lrec and (bottom layer) the surface record
 // bbp are the item's.
-template <int N, int S, bool MIX>
+// INL: the eigensolver is inlined here (k_rescue), otherwise as the compiler chooses.
+template <int N, int S, bool MIX, bool INL = false>
 __device__ __forceinline__ void layer_general(const RTWork& W, int M, int it, int layer,
                                               const typename std::conditional<MIX, float, double>::type* srec,
                                               double* lrec, double* bbp) {
@@ -206,7 +207,11 @@ __device__ __forceinline__ void layer_general(const RTWork& W, int M, int it, in
     for (int r = 0; r < n; ++r)
 #pragma unroll
       for (int c = 0; c < n; ++c) evec[r][c] = 0.0;
-    ier = asymtx_dev<n>(tol, am, evec, eval, &fail);
+    if constexpr (INL) {
+      [[clang::always_inline]] ier = asymtx_dev<n>(tol, am, evec, eval, &fail);
+    } else {
+      ier = asymtx_dev<n>(tol, am, evec, eval, &fail);
+    }
     if (fail || ier == 0) break;
   }
   if (fail || ier) { W.status[it] = 4; return; }
@@ -1226,6 +1231,26 @@ __global__ __launch_bounds__(64) void k_sabdab(RTWork W, int M0, int group) {
 }
 
 // ------------------------------------------------------------------ k_rescue
+// The kernel's first argument (and, below, its term) again, at a place that the
+// compiler does not connect with earlier uses: what a phase of a long kernel
+// needs of it is formed there instead of being held in scalar registers over
+// all phases.  Where those ran out, the compiler kept them in lanes of vector
+// registers and saved those, in lanes that were switched off as well, over
+// registers with live values of such lanes: with the eigensolver called from
+// the layers' loop, lanes without a layer came out of it with another lane
+// number, and the band solve read and wrote at wild addresses.  Hence no call
+// in that loop either, and all lanes active in it.
+__device__ __forceinline__ const RTWork& work_argument() {
+  typedef const __attribute__((address_space(4))) RTWork Arg;
+  Arg* p = (Arg*)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(p));
+  return *(const RTWork*)p;
+}
+__device__ __forceinline__ int uniform_again(int m) {
+  asm volatile("" : "+s"(m));
+  return m;
+}
+
 // The items that the symmetric path handed over (a layer without positive
 // definite S and D, a partially isolated eigenmatrix, a surface without
 // positive pivots): one wavefront takes an item through its remaining Fourier
@@ -1245,24 +1270,28 @@ __global__ __launch_bounds__(64) void k_rescue(RTWork W) {
     const int it = W.rlist[idx];
     const int L = W.L_it[it];
     for (int M = W.nfour[it] - 1; M <= W.nmoments; ++M) {
-      for (int layer = lane; layer < L; layer += 64) {
-        const double* og = W.og + ((size_t)it * km + layer) * (size_t)YO.K;
+      for (int l0 = 0; l0 < L; l0 += 64) {
+        // (lanes past the last layer repeat it: they write the same values to the
+        // same places)
+        const int layer = min(l0 + lane, L - 1), Mv = uniform_again(M);
+        const RTWork& V = work_argument();
+        const double* og = V.og + ((size_t)it * km + layer) * (size_t)YO.K;
         using T = typename std::conditional<MIX, float, double>::type;
         T* srec = reinterpret_cast<T*>(base + (size_t)layer * (2 * n * n));
         const T* Y;
-        if constexpr (MIX) Y = W.ytab;
-        else Y = W.ytab64;
+        if constexpr (MIX) Y = V.ytab;
+        else Y = V.ytab64;
 #pragma unroll 1
         for (int r = 0; r < YO.rows(); ++r) {
           T v = (T)0;
 #pragma unroll 1
-          for (int q = 0; q < YO.K; ++q) v += Y[YO.at(M, r, q)] * (T)og[q];
+          for (int q = 0; q < YO.K; ++q) v += Y[YO.at(Mv, r, q)] * (T)og[q];
           srec[r] = v;
         }
-        layer_general<N, S, MIX>(W, M, it, layer, srec, lb + (size_t)layer * LS, bb);
+        layer_general<N, S, MIX, true>(V, Mv, it, layer, srec, lb + (size_t)layer * LS, bb);
       }
       __threadfence_block();
-      const bool on = bvp_general<N, S, G>(W, M, it, lane < G, lb, LS, bb);
+      const bool on = bvp_general<N, S, G>(work_argument(), uniform_again(M), it, lane < G, lb, LS, bb);
       __threadfence_block();
       if (__ballot(lane == 0 && on) == 0ull) break;
     }

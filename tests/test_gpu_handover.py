@@ -1,0 +1,115 @@
+"""Items that leave the symmetric radiance path for the general one (k_rescue):
+after some of their Fourier terms, in lists of every length, among ordinary
+ones, and what they cost; and Fourier terms in groups of unequal size."""
+import dataclasses
+
+import numpy as np
+import pytest
+
+import oracle
+from aeroapps_amd import chem_mie as AM
+from aeroapps_amd import synthetic as S
+from aeroapps_amd import vlidort as V
+from oracle import brdf
+from oracle import chem_mie as CM
+from _fixtures import RTOL_FP64, max_rel
+from _gpu_helpers import fused
+
+pytestmark = pytest.mark.gpu
+CH = (550.0,)
+
+
+def test_resumes_at_a_later_term(gpu):
+    """A land surface whose 1 + R is positive at Fourier 0 and indefinite at
+    Fourier 1 (weights far outside those of real land): those columns go over
+    after their first term.  The mixed path at N = 8 runs every term on the
+    general path and has the same radiances within its own 1e-5."""
+    N, km, ncol, nmom = 8, 24, 13, 32
+    print(f"case resume N={N}", flush=True)
+    cols = S.make_columns(ncol, km, CH, seed=13)
+    odd, param = (1.08, 0.0497, -4.636), (2.0, 3.0)   # fiso, fgeo, fvol; Li-sparse parameters
+    x, w = np.polynomial.legendre.leggauss(N)
+    gs = np.sqrt(0.5 * w * 0.5 * (x + 1))
+    surf = brdf.vbrdf_master(N, 30.0, 40.0, 70.0, brdf.landmodis_setup(*odd, param))
+    low = [np.linalg.eigvalsh(0.5 * (a + a.T))[[0, -1]] for a in
+           (gs[:, None] * surf["F"][m] * gs * (2.0 if m == 0 else 1.0) for m in (0, 1))]
+    assert surf["ok"] and -0.98 < low[0][0] and low[0][1] < 0.995 and low[1][0] < -1.03
+    kw, par = S.make_modis_kernels(ncol, 1, seed=13)
+    marked = np.zeros(ncol, dtype=bool)
+    marked[[0, 4, 5, 11]] = True
+    kw0 = kw.copy()
+    kw[marked], par[marked] = odd, param
+    cols.sza[marked], cols.vza[marked], cols.raa[marked] = 30.0, 40.0, 70.0
+    tabs = S.make_mie_tables(CH, nmom=nmom, npol=1)
+    opt = [np.asarray(a, dtype=np.float64).T for a in
+           CM.get_aop_vector(tabs, CH, tabs[0].lambda_m, S.TRACERS, cols.qm, cols.rh, nmom, 1)[:4]]
+    f = lambda k, precision: V.scalar_landmodis(
+        cols.channels, N, False, cols.rot.T, cols.depol, *opt, cols.pe.T, cols.he.T, cols.te.T, k.T, par.T, cols.sza,
+        cols.raa, cols.vza, S.MISSING, precision=precision, return_nfourier=True)
+    I, R, br, rc, nf = f(kw, 0)
+    I1, R1, br1, rc1, nf1 = f(kw, 1)
+    assert rc == rc1 == 0 and np.isfinite(I).all() and (nf[marked] > 2).all()
+    assert np.array_equal(nf, nf1)
+    assert max_rel(I, I1) < 1.0e-5 and max_rel(R, R1) < 1.0e-5
+    plain = f(kw0, 0)
+    assert np.array_equal(I[~marked], plain[0][~marked]) and np.array_equal(nf[~marked], plain[4][~marked])
+
+
+def columns(ncol, km, seed=19):
+    """Columns of uneven height, most of them over a surface of albedo -3 or
+    1.7, whose reflection leaves pivots that are not positive at Fourier 0."""
+    cols = S.make_columns(ncol, km, CH, seed=seed, uneven_layers=(3, km))
+    rng = np.random.default_rng(5)
+    cols.albedo[0] = rng.choice([0.1, 1.7, -3.0], p=[0.2, 0.2, 0.6], size=ncol)
+    return cols
+
+
+def take(cols, pick):
+    return dataclasses.replace(cols, qm=cols.qm[pick], rh=cols.rh[pick], rot=cols.rot[:, pick], pe=cols.pe[pick],
+                               he=cols.he[pick], te=cols.te[pick], albedo=cols.albedo[:, pick], sza=cols.sza[pick],
+                               vza=cols.vza[pick], raa=cols.raa[pick], flux_factor=cols.flux_factor[pick],
+                               nlayers=cols.nlayers[pick])
+
+
+@pytest.mark.parametrize("N,ncol,precision", [(2, 10_000, 0), (3, 2500, 1), (6, 1500, 0), (9, 1100, 0)])
+def test_lists_of_every_length(gpu, N, ncol, precision):
+    """Long lists, whose items share wavefronts, give them what short ones do,
+    and that is the oracle's."""
+    import torch
+    print(f"case long list N={N} ncol={ncol} precision={precision}", flush=True)
+    cols = columns(ncol, 12)
+    tabs = S.make_mie_tables(CH, nmom=32, npol=1)
+    mie = AM.MieTables.from_synthetic(tabs)
+    rad, refl, nf = fused(torch, mie, cols, CH, N, 32, 1, nlayers=cols.nlayers, precision=precision)
+    pick = np.r_[np.arange(0, ncol, ncol // 90), ncol - 1]
+    part = take(cols, pick)
+    rad1, refl1, nf1 = fused(torch, mie, part, CH, N, 32, 1, nlayers=part.nlayers, precision=precision)
+    assert np.array_equal(rad[:, pick], rad1) and np.array_equal(refl[:, pick], refl1)
+    assert np.array_equal(nf[:, pick], nf1)
+    tau, ssa, g, pm, _ = CM.get_aop_vector(tabs, CH, tabs[0].lambda_m, S.TRACERS, part.qm, part.rh, 32, 1)
+    for c in range(0, len(pick), 5):
+        L = int(part.nlayers[c])
+        one = [np.asarray(a[c:c + 1, :, :L], dtype=np.float64) for a in (tau, ssa, g)]
+        I0, R0, nf0, _ = oracle.port().scalar_lambert(
+            L, CH, N, 32, part.rot[:, c:c + 1, :L], part.depol, *one,
+            np.asarray(pm[:, :, c:c + 1, :, :L], dtype=np.float64), part.pe[c:c + 1, :L + 1], part.he[c:c + 1, :L + 1],
+            part.te[c:c + 1, :L + 1], part.albedo[:, c:c + 1], part.sza[c:c + 1], part.raa[c:c + 1], part.vza[c:c + 1])
+        assert nf1[0, c] == nf0[0, 0]
+        assert max_rel(rad1[0, c], I0[0, 0]) < (RTOL_FP64 if precision == 0 else 1.0e-5)
+
+
+@pytest.mark.parametrize("N,nmom,ncol,precision", [(6, 32, 700, 0), (6, 32, 700, 1), (5, 32, 1300, 0), (6, 8, 5000, 0),
+                                                   (3, 5, 1900, 0), (9, 32, 250, 0)])
+def test_last_group_of_terms_is_smaller(gpu, N, nmom, ncol, precision):
+    """Numbers of columns whose Fourier terms run in groups that do not divide
+    them (5 + 5 + 2, 3 + 3 + 3 + 1, 2 + 2 + 2 + 2 + 1, 2 + 2 + 2, 16 + 2 of
+    them): the bits of columns that run all their terms in one group."""
+    import torch
+    print(f"case groups N={N} nmom={nmom} ncol={ncol}", flush=True)
+    cols = S.make_columns(ncol, 9, CH, seed=37)
+    mie = AM.MieTables.from_synthetic(S.make_mie_tables(CH, nmom=nmom, npol=1))
+    rad, refl, nf = fused(torch, mie, cols, CH, N, nmom, 1, precision=precision)
+    pick = np.r_[np.arange(0, ncol, ncol // 90), ncol - 1]
+    rad1, refl1, nf1 = fused(torch, mie, take(cols, pick), CH, N, nmom, 1, precision=precision)
+    assert np.array_equal(rad[:, pick], rad1) and np.array_equal(refl[:, pick], refl1)
+    assert np.array_equal(nf[:, pick], nf1)
