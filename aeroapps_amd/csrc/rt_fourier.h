@@ -1231,6 +1231,13 @@ __global__ __launch_bounds__(64) void k_sabdab(RTWork W, int M0, int group) {
 }
 
 // ------------------------------------------------------------------ k_rescue
+// The items that the symmetric path handed over (a layer without positive
+// definite S and D, as a forward-peaked phase function of as few moments as
+// streams has; a partially isolated eigenmatrix; a surface without positive
+// pivots; optics that are no numbers), through their remaining Fourier terms on
+// the general path.  Launched once per chunk after the symmetric path's terms;
+// mostly the list is empty and the launch then ends at once.
+
 // The kernel's first argument (and, below, its term) again, at a place that the
 // compiler does not connect with earlier uses: what a phase of a long kernel
 // needs of it is formed there instead of being held in scalar registers over
@@ -1251,49 +1258,116 @@ __device__ __forceinline__ int uniform_again(int m) {
   return m;
 }
 
-// The items that the symmetric path handed over (a layer without positive
-// definite S and D, a partially isolated eigenmatrix, a surface without
-// positive pivots): one wavefront takes an item through its remaining Fourier
-// terms on the general path, the layers across the lanes, then the band solve.
-// Launched once per chunk after the symmetric path's terms; the list is empty
-// for physical inputs and the launch then ends at once.
-template <int N, int S, bool MIX>
-__global__ __launch_bounds__(64) void k_rescue(RTWork W) {
-  constexpr int n = N * S, G = bvp_group(n);
+// SAB/DAB of one layer: rows of the contraction table Y times og.
+template <int N, int S, class T>
+__device__ __forceinline__ void sabdab_rows(const T* __restrict__ Y, const double* __restrict__ og,
+                                            T* __restrict__ srec) {
   constexpr YOff YO(N, S);
-  const int lane = threadIdx.x;
+  constexpr int RB = 8, K = YO.K, ROWS = YO.rows();
+#pragma unroll 1
+  for (int r0 = 0; r0 < ROWS; r0 += RB) {
+    T v[RB];
+#pragma unroll
+    for (int i = 0; i < RB; ++i) v[i] = (T)0;
+    // (the last block's rows beyond the table repeat its last row)
+#pragma unroll 2
+    for (int q = 0; q < K; ++q) {
+      const T o = (T)og[q];
+#pragma unroll
+      for (int i = 0; i < RB; ++i) v[i] += Y[(ROWS % RB == 0 ? r0 + i : min(r0 + i, ROWS - 1)) * K + q] * o;
+    }
+#pragma unroll
+    for (int i = 0; i < RB; ++i)
+      if (ROWS % RB == 0 || r0 + i < ROWS) srec[r0 + i] = v[i];
+  }
+}
+
+// One wavefront takes up to RESCUE_ITEMS items through their terms together:
+// their (item, layer) pairs fill its lanes, then the band solve takes 64 / G of
+// them at a time.  A short list gets a wavefront per item until there is one for
+// each SIMD.  Records are in abuf, which the symmetric path no longer needs.
+// With one item per wavefront, and few wavefronts, 72 layers took two rounds of
+// 64 lanes and the band solve 8 of them.  Calls whose columns all go over
+// (albedo 1.7), N = 6, that kernel / the general path for every column from the
+// start / now: 20,000 columns 213.8 / 27.4 / 37.3 ms, 5,000 - / 11.5 / 11.1, 64
+// - / 6.3 / 5.8, one - / 5.2 / 4.9; optics that are no numbers in every column:
+// 20,000 at N = 6 31.9 / 14.4 / 19.6, 1,200 at N = 12 85 / 25.4 / 17.1, 2,000 at
+// N = 4 with three Stokes components 107 / 35.8 / 21.4.  (Long lists stay above
+// the general path's time where a wavefront waits for the slowest of its items;
+// a tenth of the columns costs 1.4 ms beside 7.9.)  Two wavefronts per SIMD up
+// to n = 4 (50,000 columns at N = 4 37.2 -> 32.5 ms); at n = 6 they spill 1.4 KB
+// a lane (5,000 columns 11.0 -> 14.3).
+template <int N, int S, bool MIX>
+__global__ __launch_bounds__(64, (N * S <= 4) ? 2 : 1) void k_rescue(RTWork W) {
+  constexpr int n = N * S, G = bvp_group(n), IPW = 64 / G;
+  constexpr YOff YO(N, S);
+  static_assert(RESCUE_ITEMS <= 8, "an item per lane, at most eight readlanes each");
+  const int lane = threadIdx.x, g = lane / G;
   const int count = *W.rcnt, km = W.km, LS = LOff(N, S).size();
-  double* base = W.rbuf + (size_t)blockIdx.x * rescue_doubles(N, S, km);
-  double* lb = base + (size_t)km * (2 * n * n);
-  double* bb = lb + (size_t)km * LS;
-  for (int idx = blockIdx.x; idx < count; idx += gridDim.x) {
-    const int it = W.rlist[idx];
-    const int L = W.L_it[it];
-    for (int M = W.nfour[it] - 1; M <= W.nmoments; ++M) {
-      for (int l0 = 0; l0 < L; l0 += 64) {
-        // (lanes past the last layer repeat it: they write the same values to the
+  if (count == 0) return;
+  const int ipw = min(RESCUE_ITEMS, (count + RESCUE_WAVES - 1) / RESCUE_WAVES);
+  const int nb = min((int)gridDim.x, max(1, W.rcap / ipw));
+  if ((int)blockIdx.x >= nb) return;
+  const size_t stride = rescue_doubles(N, S, km);
+  double* base = W.abuf + (size_t)blockIdx.x * ipw * stride;
+  for (int c0 = blockIdx.x * ipw; c0 < count; c0 += nb * ipw) {
+    // lane j < ni: item j, its layers and its next term
+    const int ni = min(ipw, count - c0);
+    const int itl = lane < ni ? W.rlist[c0 + lane] : 0;
+    const int Ll = lane < ni ? W.L_it[itl] : 0;
+    const int Ml = lane < ni ? W.nfour[itl] - 1 : W.nmoments;
+    int M = W.nmoments;
+    for (int j = 0; j < ni; ++j) M = min(M, __builtin_amdgcn_readlane(Ml, j));
+    unsigned todo = (1u << ni) - 1u;
+    for (; M <= W.nmoments && todo != 0u; ++M) {
+      const unsigned now = todo & (unsigned)__ballot(Ml <= M);
+      if (now == 0u) continue;
+      int total = 0;
+      for (unsigned m = now; m != 0u; m &= m - 1u) total += __builtin_amdgcn_readlane(Ll, __ffs(m) - 1);
+      for (int p0 = 0; p0 < total; p0 += 64) {
+        // (lanes past the last pair repeat it: they write the same values to the
         // same places)
-        const int layer = min(l0 + lane, L - 1), Mv = uniform_again(M);
+        const int p = min(p0 + lane, total - 1);
+        int j = 0, layer = 0, acc = 0;
+        for (unsigned m = now; m != 0u; m &= m - 1u) {
+          const int b = __ffs(m) - 1, Lb = __builtin_amdgcn_readlane(Ll, b);
+          if (p >= acc) { j = b; layer = p - acc; }
+          acc += Lb;
+        }
+        const int it = __shfl(itl, j, 64);
         const RTWork& V = work_argument();
-        const double* og = V.og + ((size_t)it * km + layer) * (size_t)YO.K;
+        const int Mv = uniform_again(M);
         using T = typename std::conditional<MIX, float, double>::type;
-        T* srec = reinterpret_cast<T*>(base + (size_t)layer * (2 * n * n));
+        double* rec = base + (size_t)j * stride;
+        T* srec = reinterpret_cast<T*>(rec + (size_t)layer * (2 * n * n));
+        double* lb = rec + (size_t)km * (2 * n * n);
         const T* Y;
         if constexpr (MIX) Y = V.ytab;
         else Y = V.ytab64;
-#pragma unroll 1
-        for (int r = 0; r < YO.rows(); ++r) {
-          T v = (T)0;
-#pragma unroll 1
-          for (int q = 0; q < YO.K; ++q) v += Y[YO.at(Mv, r, q)] * (T)og[q];
-          srec[r] = v;
-        }
-        layer_general<N, S, MIX, true>(V, Mv, it, layer, srec, lb + (size_t)layer * LS, bb);
+        sabdab_rows<N, S, T>(Y + YO.at(Mv, 0, 0), V.og + ((size_t)it * km + layer) * (size_t)YO.K, srec);
+        layer_general<N, S, MIX, true>(V, Mv, it, layer, srec, lb + (size_t)layer * LS, lb + (size_t)km * LS);
       }
       __threadfence_block();
-      const bool on = bvp_general<N, S, G>(work_argument(), uniform_again(M), it, lane < G, lb, LS, bb);
+      for (unsigned rest = now; rest != 0u;) {
+        // lane group g: the g-th item of the rest
+        int mine = -1, first = __ffs(rest) - 1;
+        unsigned m = rest;
+#pragma unroll 1
+        for (int q = 0; q < IPW && m != 0u; ++q, m &= m - 1u)
+          if (g == q) mine = __ffs(m) - 1;
+        const int j = mine >= 0 ? mine : first;
+        const int it = __shfl(itl, j, 64);
+        const double* lb = base + (size_t)j * stride + (size_t)km * (2 * n * n);
+        const bool on = bvp_general<N, S, G>(work_argument(), uniform_again(M), it, mine >= 0, lb, LS, lb + (size_t)km * LS);
+        // an item that is done leaves
+        const unsigned long long goes = __ballot(on);
+        m = rest;
+#pragma unroll 1
+        for (int q = 0; q < IPW && m != 0u; ++q, m &= m - 1u)
+          if (((goes >> (q * G)) & 1ull) == 0ull) todo &= ~(m & (0u - m));
+        rest = m;
+      }
       __threadfence_block();
-      if (__ballot(lane == 0 && on) == 0ull) break;
     }
   }
 }
@@ -1334,7 +1408,7 @@ int fourier_loop_sym(const RTWork& W, int nitems, int* const lists[2], int* coun
     }
   }
   prof_begin(PROF_BVP, st);
-  hipLaunchKernelGGL((k_rescue<N, S, MIX>), dim3(W.rblocks), dim3(64), 0, st, W);
+  hipLaunchKernelGGL((k_rescue<N, S, MIX>), dim3(rescue_grid(W)), dim3(64), 0, st, W);
   prof_end(PROF_BVP, st);
   AA_CHECK(hipGetLastError());
   return 0;

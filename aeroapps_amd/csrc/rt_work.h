@@ -6,6 +6,8 @@
 // ([it][layer][field]) so that the wavefront solving one item reads its layer
 // data contiguously.
 #pragma once
+#include <algorithm>
+
 #include "aa_common.h"
 
 namespace aa {
@@ -133,11 +135,10 @@ struct RTWork {
   double* bbuf = nullptr;          // [it][bstride] surface terms of the bottom layer
   int lstride = 0, bstride = 0;
   // items of the symmetric path that continue on the general path (k_rescue):
-  // list, count, and one item's records per workgroup
+  // list, count, and how many items' records abuf holds at a time
   int* rlist = nullptr;
   int* rcnt = nullptr;
-  int rblocks = 0;
-  double* rbuf = nullptr;          // [rblocks][rescue_doubles]
+  int rcap = 0;
   // ---- quadrature and PI tables of the quadrature streams (device)
   const double* quad = nullptr;    // QOff: [qs N][qw N][xq: M][l][i][S][S][scalings]
   const double* phi = nullptr;     // the same layout, xq times sqrt(w_i/mu_i)
@@ -358,10 +359,19 @@ struct QOff {
 };
 
 
-// Doubles of one workgroup's records in k_rescue: SAB/DAB, layer solutions and
-// surface terms of one item.
+// Doubles of one item's records in k_rescue: SAB/DAB, layer solutions and
+// surface terms.
 __host__ __device__ constexpr size_t rescue_doubles(int N, int S, int km) {
   return (size_t)km * (2 * N * S * N * S + LOff(N, S).size()) + BOff(N, N * S, S).size();
+}
+
+// Items that a wavefront of k_rescue takes together, and the wavefronts among
+// which a list is spread before any gets a second item (the SIMDs of the GPU:
+// the kernel's registers allow one wavefront on each).
+constexpr int RESCUE_ITEMS = 8, RESCUE_WAVES = 1024;
+inline unsigned rescue_grid(const RTWork& W) {
+  const int want = std::max(std::min(W.cap, RESCUE_WAVES), (W.cap + RESCUE_ITEMS - 1) / RESCUE_ITEMS);
+  return (unsigned)std::min(std::min(want, W.rcap), 4 * RESCUE_WAVES);
 }
 
 // Launch shapes of the Fourier-term kernels.  Lanes per item of the band

@@ -347,15 +347,16 @@ size_t carve_work(Carver& C, RTWork& W, int cap) {
   const bool sym = sym_path(W.N, W.S, mixed);
   W.astride = AOff(W.N, W.S).size();
   if (sym) {
-    W.abuf = C.take<double>((size_t)cap * km * W.astride * W.terms);
+    // k_rescue's records follow the modes in the same memory: at least half of the
+    // chunk's items at a time, and all of a handful
+    const size_t rec = rescue_doubles(W.N, W.S, km);
+    const size_t pool = std::max((size_t)cap * km * W.astride * W.terms, (size_t)std::min(cap, RESCUE_ITEMS) * rec);
+    W.abuf = C.take<double>(pool);
+    W.rcap = (int)std::min(pool / rec, (size_t)cap);
     W.cums = C.take<double>((size_t)cap * W.terms * W.S);
     W.tflag = C.take<int>((size_t)cap * W.terms);
     W.pis = C.take<double>((size_t)cap * PiOff(W.N, W.S).size());
     W.rlist = C.take<int>(cap);
-    // workgroups of k_rescue: up to 512, fewer for small chunks, so that their
-    // records add at most an eighth of an item's general-path records to each item
-    W.rblocks = std::min(512, (cap + 7) / 8);
-    W.rbuf = C.take<double>((size_t)W.rblocks * rescue_doubles(W.N, W.S, km));
   } else {
     W.lbuf = C.take<double>((size_t)cap * km * W.lstride);
     W.bbuf = C.take<double>((size_t)cap * W.bstride);
@@ -370,10 +371,9 @@ size_t carve_work(Carver& C, RTWork& W, int cap) {
 
 size_t bytes_per_item(const RTWork& W0) {
   RTWork W = W0;
-  // (8 items share one rescue workgroup)
   Carver a(nullptr), b(nullptr);
-  size_t s1 = carve_work(a, W, 8), s2 = carve_work(b, W, 16);
-  return (s2 - s1 + 7) / 8 + 256 * 24;
+  size_t s1 = carve_work(a, W, 1024), s2 = carve_work(b, W, 2048);
+  return (s2 - s1 + 1023) / 1024 + 256 * 24;
 }
 
 // Items of one work chunk of W's shape on the current GPU: the work budget
@@ -434,8 +434,7 @@ int run_items(RTWork W, int g0, int g1, hipStream_t st, const int* d_items = nul
   const size_t tab_bytes = qtab.size() * sizeof(double) + std::max<size_t>(1, ytab.size()) * sizeof(float) +
                            std::max<size_t>(1, ytab64.size()) * sizeof(double) +
                            std::max<size_t>(1, btab.size()) * sizeof(double) +
-                           sizeof(int) * ((LBINS + 1) * (W.nmoments + 2) + 1) +
-                           rescue_doubles(W.N, W.S, W.km) * sizeof(double) + 16 * 256;
+                           sizeof(int) * ((LBINS + 1) * (W.nmoments + 2) + 1) + 16 * 256;
   // Fourier terms per group: as many as the batch's size calls for, one where
   // a group's records would not leave the batch in one chunk
   W.terms = term_group(nitems, W.nmoments);

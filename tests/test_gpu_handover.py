@@ -113,3 +113,33 @@ def test_last_group_of_terms_is_smaller(gpu, N, nmom, ncol, precision):
     rad1, refl1, nf1 = fused(torch, mie, take(cols, pick), CH, N, nmom, 1, precision=precision)
     assert np.array_equal(rad[:, pick], rad1) and np.array_equal(refl[:, pick], refl1)
     assert np.array_equal(nf[:, pick], nf1)
+
+
+def test_handed_over_items_run_side_by_side(gpu):
+    """What a call costs when its columns go over: 64 of them, which fit the GPU
+    at once, no more than three times one (1.2; item after item, eight to a
+    wavefront, 8); 20,000 no more than nine times as many ordinary ones (4.7; a
+    wavefront for each, 27)."""
+    import torch
+    from perf import cases
+    print("case cost of handed-over items", flush=True)
+
+    def cost(ncol, albedo):
+        state = cases.prepare(cases._case("", "fused", ncol, 1, 6, nmom=32), 3)
+        state["albedo"][:] = albedo
+        cases.run(state)
+        best = np.inf
+        for _ in range(3):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            cases.run(state)
+            b.record()
+            b.synchronize()
+            best = min(best, a.elapsed_time(b))
+        return best
+
+    one, many = cost(1, 1.7), cost(64, 1.7)
+    plain, over = cost(20_000, 0.1), cost(20_000, 1.7)
+    print(f"1: {one:.2f} ms, 64: {many:.2f}; 20,000 ordinary: {plain:.2f}, handed over: {over:.2f}", flush=True)
+    assert many < 3.0 * one
+    assert over < 9.0 * plain
