@@ -36,6 +36,7 @@ SIGNATURES = {
     "aa_set_tuning": (_ci, [_ci, _ci, _ci, _vp]),
     "aa_get_tuning": (_ci, [_ci, _ci, _ci, _vp]),
     "aa_load_tuning": (_ci, [_cp]),
+    "aa_tuning_live": (_ci, [_ci, _ci, _ci, _ip, _ip]),
     "aa_mie_create_rc": (_ci, [ctypes.POINTER(_vp), _cp, _ci, _cp, _ip, _vp, _vp, _ip]),
     "aa_mie_destroy": (_ci, [_vp]),
     "aa_get_aop_vector": (_ci, [_vp, _ci, _ci, _ci, _ci, _fp, _cp, _ci, _fp, _fp, _ci, _ci, _fp, _fp, _fp, _fp, _ip]),

@@ -130,4 +130,15 @@ int aa_load_tuning(const char* path) {
   return r == -1 ? AA_ENOFILE : (r == -2 ? AA_EARG : 0);
 }
 
+int aa_tuning_live(int nstreams, int nstokes, int precision, int* bvp_lanes, int* sab_pairs) {
+  using namespace aa;
+  if (!bvp_lanes || !sab_pairs || nstreams < 1 || (nstokes != 1 && nstokes != 3) || (precision != 0 && precision != 1))
+    return AA_EARG;
+  const int n = nstreams * nstokes;
+  const bool mixed = precision == 1;
+  *bvp_lanes = !sym_path(nstreams, nstokes, mixed) && bvp_group_alt(n) != bvp_group(n);
+  *sab_pairs = needs_sabdab(nstreams, nstokes, mixed) && sab_groups_alt(nstreams, nstokes) != sab_groups(nstreams, nstokes);
+  return 0;
+}
+
 }  // extern "C"

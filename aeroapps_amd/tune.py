@@ -3,10 +3,11 @@
 For each (streams, Stokes, precision) class it times the fused device path
 (``aa_column_radiance_dev``) on a seeded sample with every launch shape this
 build has -- the band solver's lanes per item (``bvp_lanes``) and the SAB/DAB
-kernel's (item, layer) pairs per wavefront (``sab_pairs``) -- keeps the
-fastest, and writes the table the library reads at start-up
-(``aeroapps_amd/tuning_gfx950.txt``; format in include/aeroapps_amd.h).  All
-shapes give bit-identical results; the tuner checks that too.
+kernel's (item, layer) pairs per wavefront (``sab_pairs``), as far as the class
+runs those kernels (``live``) -- keeps the fastest, and writes the table the
+library reads at start-up (``aeroapps_amd/tuning_gfx950.txt``; format in
+include/aeroapps_amd.h).  All shapes give bit-identical results; the tuner
+checks that too.
 
     python -m aeroapps_amd.tune [--ncol 20000] [--out aeroapps_amd/tuning_gfx950.txt]
 """
@@ -66,6 +67,15 @@ def shape_candidates(nstreams: int, nstokes: int) -> List[Tuple[int, int]]:
             out.add((got["bvp_lanes"], got["sab_pairs"]))
     set_tuning(nstreams, nstokes, 0, **orig)
     return sorted(out)
+
+
+def live(nstreams: int, nstokes: int, precision: int) -> Tuple[bool, bool]:
+    """Whether bvp_lanes and sab_pairs change what the class launches: not where
+    it runs on the symmetric path (sab_pairs: in FP64), nor with one shape."""
+    b, s = ctypes.c_int(), ctypes.c_int()
+    _lib.check(_lib.lib().aa_tuning_live(nstreams, nstokes, precision, ctypes.byref(b), ctypes.byref(s)),
+               "aa_tuning_live")
+    return bool(b.value), bool(s.value)
 
 
 class Sample:
@@ -128,18 +138,27 @@ def tune_class(torch, nstreams: int, nstokes: int, precisions: Sequence[int], nc
         for prec in precisions:
             times = {}
             ref = None
+            clear_tuning(nstreams, nstokes, prec)
+            default = get_tuning(nstreams, nstokes, prec)
+            bvp, sab = live(nstreams, nstokes, prec)
             for g, p in shape_candidates(nstreams, nstokes):
-                set_tuning(nstreams, nstokes, prec, g, p, 0)
+                shape = (g if bvp else default["bvp_lanes"], p if sab else default["sab_pairs"])
+                if shape in times:                         # the same launches as one already timed
+                    times[(g, p)] = times[shape]
+                    continue
+                set_tuning(nstreams, nstokes, prec, *shape, 0)
                 smp.run(prec)                              # warm-up (arena, tables)
                 t = min(smp.run(prec) for _ in range(reps))
                 res = smp.outputs()
                 if ref is None:
                     ref = res
                 elif not (np.array_equal(res[0], ref[0]) and np.array_equal(res[1], ref[1])):
-                    raise RuntimeError(f"shape {(g, p)} changed the results of N={nstreams} S={nstokes}")
-                times[(g, p)] = t
-                log(f"N={nstreams} S={nstokes} precision={prec} bvp_lanes={g} sab_pairs={p}: {t * 1e3:.1f} ms")
-            best = min(times, key=times.get)
+                    raise RuntimeError(f"shape {shape} changed the results of N={nstreams} S={nstokes}")
+                times[shape] = times[(g, p)] = t
+                log(f"N={nstreams} S={nstokes} precision={prec} bvp_lanes={shape[0]} sab_pairs={shape[1]}: "
+                    f"{t * 1e3:.1f} ms")
+            # (of shapes that launch the same, the default)
+            best = min(times, key=lambda s: (times[s], s[0] != default["bvp_lanes"], s[1] != default["sab_pairs"]))
             clear_tuning(nstreams, nstokes, prec)
             out[prec] = (best, times)
     finally:
@@ -153,7 +172,9 @@ def write_table(path: str, results: Dict[Tuple[int, int], Dict[int, tuple]], nco
              "# nstreams nstokes precision bvp_lanes sab_pairs chunk_items"]
     for (N, Sx), per in sorted(results.items()):
         for prec, (best, times) in sorted(per.items()):
-            alt = "  ".join(f"{g}/{p}:{t * 1e3:.1f}" for (g, p), t in sorted(times.items()))
+            bvp, sab = live(N, Sx, prec)
+            alt = "  ".join(f"{g}/{p}:{t * 1e3:.1f}" for (g, p), t in sorted(times.items())
+                            if (bvp or g == best[0]) and (sab or p == best[1]))
             lines.append(f"{N} {Sx} {prec} {best[0]} {best[1]} 0   # {alt}")
     with open(path, "w") as fh:
         fh.write("\n".join(lines) + "\n")

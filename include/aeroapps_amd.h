@@ -527,6 +527,10 @@ typedef struct aa_tuning {
 int aa_set_tuning(int nstreams, int nstokes, int precision, const aa_tuning* t);
 int aa_get_tuning(int nstreams, int nstokes, int precision, aa_tuning* t);
 int aa_load_tuning(const char* path);
+/* Whether a class runs kernels whose shape bvp_lanes (sab_pairs) chooses, with
+ * more than one shape: 1 or 0.  The symmetric path has no band solver and, in
+ * FP64, no SAB/DAB kernel; a choice for it is accepted and changes nothing. */
+int aa_tuning_live(int nstreams, int nstokes, int precision, int* bvp_lanes, int* sab_pairs);
 
 /* Library version string. */
 const char* aa_version(void);
