@@ -25,6 +25,13 @@ def _ptr(a, kind=_dp):
     return a.ctypes.data_as(kind)
 
 
+def _check_number(*arrs):
+    """Raises as _f64 does where an argument is no array of numbers, without its copy."""
+    for a in arrs:
+        if np.asarray(a).dtype.kind not in "fiub":
+            _f64(a)
+
+
 def _all_f32(*arrs):
     return all(isinstance(a, np.ndarray) and a.dtype == np.float32 and a.flags.f_contiguous for a in arrs)
 
@@ -56,6 +63,7 @@ def scalar_lambert(channels, nstreams, plane_parallel, ROT, depol, tau, ssa, g, 
     Layer optics that are float32 in Fortran order, as get_aop_vector returns
     them, go to the device as they are and are widened there."""
     if _all_f32(tau, ssa, pmom) and tau.ndim == 3 and ssa.shape == tau.shape and pmom.shape[:3] == tau.shape:
+        _check_number(channels, g, pe, te)   # (not read)
         return _scalar_lambert_f32(nstreams, plane_parallel, ROT, depol, tau, ssa, pmom, he, albedo, solar_zenith,
                                    relat_azymuth, sensor_zenith, MISSING, precision, return_nfourier)
     channels, ROT, depol, tau, ssa, g, pmom, pe, he, te, albedo, sza, raa, vza = map(
