@@ -10,9 +10,10 @@ enum ProfKind {
   PROF_GEOM,        // Chapman + first-order sun paths
   PROF_ITEM,        // per-column recursions
   PROF_LAYER,       // per-layer eigensystem + particular solutions
-  PROF_BVP,         // band LU + back-substitution + source + convergence
+  PROF_BVP,         // boundary-value problem + source (general path: + convergence)
   PROF_BRDF,        // BRDF supplement (MODIS land surface)
-  PROF_SABDAB,      // FP32 SAB/DAB contraction of the mixed path (matrix cores)
+  PROF_SABDAB,      // SAB/DAB contraction (matrix cores)
+  PROF_CONVERGE,    // convergence test of the symmetric path, and the items it hands over
   PROF_KINDS
 };
 bool prof_on();

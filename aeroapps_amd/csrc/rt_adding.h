@@ -28,12 +28,13 @@
 // pairs per lane and no LDS.
 //
 // Bound: the dependent chain of the 2n pivots (broadcast, reciprocal, row
-// update) per layer for small batches, the records' bytes (832 per layer at
-// N = 6) for large ones.  Measured against the pivoted band solve (k_bvp, 8 or
-// 32 lanes per item): N = 6, 400,000 items 204 -> 49 ms (2.5 TB/s of records);
-// one item 4.3 ms over its terms -> 0.13 ms (all terms side by side); N = 12,
-// 1,200 items 15.5 -> 1.3 ms; three Stokes components N = 4, 16,000 items 133 ->
-// 6.3 ms.
+// update) per layer for small batches, the FP64 issue for large ones (N = 6: VALU
+// busy four fifths of the time at three wavefronts per SIMD; an item and term
+// read 66.8 KB, 832 bytes per layer and the beam's fields, 2.9 TB/s).  Measured
+// against the pivoted band solve (k_bvp, 8 or 32 lanes per item): N = 6, 400,000
+// items 204 -> 47 ms; one item 4.3 ms over its terms -> 0.13 ms (all terms side
+// by side); N = 12, 1,200 items 15.5 -> 1.3 ms; three Stokes components N = 4,
+// 16,000 items 133 -> 6.3 ms.
 #pragma once
 #include <type_traits>
 #include "rt_work.h"

@@ -1,5 +1,5 @@
-// Fourier convergence of one item, shared by the boundary-value kernels of the
-// symmetric path (k_adding) and of the general path (k_bvp, k_rescue).
+// Fourier convergence of one item, shared by the symmetric path (k_converge) and
+// the general path (k_bvp, k_rescue).
 #pragma once
 #include "rt_work.h"
 

@@ -1399,17 +1399,19 @@ int fourier_loop_sym(const RTWork& W, int nitems, int* const lists[2], int* coun
     prof_end(PROF_LAYER, st);
     prof_begin(PROF_BVP, st);
     hipLaunchKernelGGL((k_adding<N, S, MIX>), dim3(nb, ng), dim3(64), 0, st, W, M, in, counts + j * LBINS);
+    prof_end(PROF_BVP, st);
+    prof_begin(PROF_CONVERGE, st);
     hipLaunchKernelGGL((k_converge<N, S>), dim3(nc), dim3(64), 0, st, W, M, (int)ng, in, counts + j * LBINS, out,
                        counts + (j + 1) * LBINS, W.lcnt + j + 1);
-    prof_end(PROF_BVP, st);
+    prof_end(PROF_CONVERGE, st);
     if (mid && M + (int)ng > std::min(W.mid_term, W.nmoments)) {
       AA_CHECK(hipEventRecord(W.mid_event, st));
       mid = false;
     }
   }
-  prof_begin(PROF_BVP, st);
+  prof_begin(PROF_CONVERGE, st);
   hipLaunchKernelGGL((k_rescue<N, S, MIX>), dim3(rescue_grid(W)), dim3(64), 0, st, W);
-  prof_end(PROF_BVP, st);
+  prof_end(PROF_CONVERGE, st);
   AA_CHECK(hipGetLastError());
   return 0;
 }

@@ -45,8 +45,10 @@
 // 201 -> 58 ms (127 with the records stored straight from the lanes), mixed,
 // 240,004 items 110 -> 63 ms (168); three Stokes components N = 4, 16,000 items
 // 361 -> 17.2 ms (k_modes_pair; a lane per layer, its matrix partly in scratch,
-// took 33 and 12 for the triangles from k_sabdab).  At N = 6 the records are
-// written at 2.1 TB/s and the VALU issues 5.5k instructions per wavefront.
+// took 33 and 12 for the triangles from k_sabdab).  At N = 6 FP64 an item and
+// term write 65.4 KB (its records are 59.9), 2.3 TB/s at 400,000 items, and read
+// 27.6; a wavefront issues 6.8k VALU instructions, which keep the VALU busy half
+// of the time.
 #pragma once
 #include <type_traits>
 #include "rt_work.h"

@@ -31,13 +31,14 @@ METRIC = "columns/sec at 72 layers/12 streams, mixed vs FP64 GPU; p99 granule la
 PEAK_FP64_TFLOPS = 78.6
 PEAK_FP32_MFMA_TFLOPS = 157.3
 PEAK_HBM_GBS = 8000.0
-PROF_NAMES = ["mie", "check", "optics", "geom", "item", "layer", "bvp", "brdf", "sabdab"]
-# Bytes per item-term (read, written) of the radiance kernels at N=6 scalar and
-# 72 layers, keyed (kernel, N, S, mixed): the layer records of 90 doubles that
-# k_modes writes and k_adding reads, with the coefficients (and in the mixed
-# path the FP32 SAB/DAB block) and transmittances that they are made from
-TRAFFIC_PER_ITEM_TERM = {("bvp", 6, 1, False): (56.4e3, 0.1e3), ("bvp", 6, 1, True): (56.4e3, 0.1e3),
-                         ("layer", 6, 1, False): (11.5e3, 51.8e3), ("layer", 6, 1, True): (32.3e3, 51.8e3)}
+PROF_NAMES = ["mie", "check", "optics", "geom", "item", "layer", "bvp", "brdf", "sabdab", "converge"]
+# HBM bytes per item-term (read, written) of the radiance kernels at N=6 scalar
+# and 72 layers, keyed (kernel, N, S, mixed), from FETCH_SIZE/WRITE_SIZE counter
+# runs scaled by a copy-kernel calibration
+# (profiles/hbm_traffic_40k_columns_4ch_12streams.md); the layer records alone
+# are 72 x 104 doubles, 59.9 KB
+TRAFFIC_PER_ITEM_TERM = {("bvp", 6, 1, False): (66.8e3, 0.0), ("bvp", 6, 1, True): (64.9e3, 0.0),
+                         ("layer", 6, 1, False): (27.6e3, 65.4e3), ("layer", 6, 1, True): (33.6e3, 62.3e3)}
 
 
 def symmetric(N, S_, mixed):
@@ -315,7 +316,7 @@ def main():
         msa = (ctypes.c_double * nk)()
         lna = (ctypes.c_longlong * nk)()
         _lib.check(L.aa_profile_read(msa, lna, nk), "aa_profile_read")
-        keep = [k for k in range(nk) if k < 7 or (k == 7 and modis) or (k == 8 and lna[k] > 0)]
+        keep = [k for k in range(nk) if k < 7 or (k == 7 and modis) or (k >= 8 and lna[k] > 0)]
         kms = {PROF_NAMES[k]: msa[k] for k in keep}
         kln = {PROF_NAMES[k]: lna[k] for k in keep}
         ms_per_step = el * 1000.0 / args.steps
@@ -381,9 +382,9 @@ def main():
         """FP64-VALU roofline of one radiance kernel over the timed region:
         algorithmic flops (F_b for k_modes or k_layer, F_c + F_d for k_adding
         or k_bvp) over the kernel's total HIP-event time; traffic per launch
-        from the record sizes."""
+        from the counter constants."""
         sym = symmetric(N or max(wl["stream_choices"]), Sx, rmx is not None)
-        shown = {"layer": "modes", "bvp": "adding"}[kname] if sym else kname
+        shown = {"layer": "modes" if (N or 1) * Sx <= 8 else "modes_pair", "bvp": "adding"}[kname] if sym else kname
         ms = kms[kname]
         launches = max(1, kln[kname])
         flops = fb if kname == "layer" else fc + fd
@@ -429,8 +430,8 @@ def main():
                                f"{'vector' if vector else 'scalar'} "
                                f"{'MODIS land BRDF (Lambertian + Ross-thick + Li-sparse)' if modis else 'Lambertian'}",
                    "precision": "mixed (FP32 Chem_Mie optics, FP32 phase-matrix contraction on MFMA, FP32 source "
-                                "assembly from 8 streams on; FP64 eigensystem and boundary-value elimination; the "
-                                "FP64 line is FP64 throughout with an FP64 MFMA contraction)"
+                                "assembly from 8 streams per hemisphere on; FP64 eigensystem and boundary-value "
+                                "problem; the FP64 line is FP64 throughout)"
                                 if rmx is not None else "fp64",
                    "path": ("aa_column_radiance_modis_dev" if modis else "aa_column_radiance_dev") +
                            " (Chem_Mie optics + VLIDORT radiance, device-resident)",

@@ -542,8 +542,9 @@ const char* aa_version(void);
  * milliseconds and launch counts for nkinds classes (0 Chem_Mie optics,
  * 1 input checks, 2 layer optics/delta-M, 3 Chapman + first-order geometry,
  * 4 per-column setup, 5 per-layer eigensystems, 6 boundary-value problem +
- * source + convergence, 7 BRDF supplement, 8 the mixed path's SAB/DAB
- * contraction on the matrix cores) and switches recording off. */
+ * source, 7 BRDF supplement, 8 the SAB/DAB contraction on the matrix cores,
+ * 9 convergence test of the symmetric path and the items it hands over; the
+ * general path's test is part of 6) and switches recording off. */
 int aa_profile_start(void);
 int aa_profile_read(double* ms, long long* launches, int nkinds);
 
