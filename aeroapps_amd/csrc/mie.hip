@@ -481,14 +481,23 @@ int launch_get_aop(const aa_mie* t, int km, int nobs, int nch, int nq, const int
   if (ntr_eff > MAXTR || blocks > 0x7fffffffL) return -1;
   // table rows are addressed with 32-bit row indices
   if ((long)t->dev.ntracer * t->dev.nch * t->dev.nrh > 0x7fffffffL) return -1;
-  // The layer chunks do not depend on each other: up to 32,768 (column,
-  // channel) pairs each has its own wavefront (one column: 322 -> 51 us; 8,000
-  // columns x 2 channels, six moment sets: 5.1 -> 4.7 ms).  Larger batches fill
-  // the GPU anyhow and a wavefront walks its column's chunks (400,000 pairs:
-  // 28.5 ms, apart 30.1).
+  // four moments per lane where rows, moments and the table base come in whole
+  // aligned groups of four and element offsets fit 32 bits
+  const long elems = (long)t->dev.ntracer * t->dev.nch * t->dev.nrh * t->dev.npol * t->dev.nmom;
+  const bool v4 = d_pmom && nmom % 4 == 0 && t->dev.nmom % 4 == 0 && ((size_t)t->dev.pmom & 15) == 0 &&
+                  elems <= 0x7fffffffL;
+  // The layer chunks do not depend on each other: in smaller batches each has its
+  // own wavefront, larger ones fill the GPU anyhow and a wavefront walks its
+  // column's chunks.  (Column, channel) pairs, apart / walked, us: 64 moments 1
+  // 13 / 96, 1,000 44 / 111, 16,000 605 / 637, 24,000 959 / 961, 32,000 1,291 /
+  // 1,273, 64,000 2,693 / 2,485, 400,000 17,473 / 16,080; six sets of 32 16,000
+  // 1,447 / 1,479, 24,000 2,212 / 2,202, 32,000 3,083 / 2,946; 30 moments, one a
+  // lane, 32,000 1,986 / 2,082, 40,000 2,521 / 2,563, 64,000 4,072 / 4,025; no
+  // moments 12,000 181 / 187, 16,000 248 / 245, 32,000 498 / 477.
+  const long apart = !d_pmom ? 16384 : (v4 ? 24576 : 49152);
   const int kc = std::max(1, std::min(MIE_KC_MAX, MIE_CAP / std::max(1, ntr_eff)));
   // (a grid's second dimension ends at 65,536; a wavefront then walks several)
-  const int ny = blocks <= 32768 ? std::min((km + kc - 1) / kc, 65536) : 1;
+  const int ny = blocks <= apart ? std::min((km + kc - 1) / kc, 65536) : 1;
   prof_begin(PROF_MIE, st);
   const dim3 grid((unsigned)blocks, (unsigned)ny);
   auto launch = [&](auto w4) {
@@ -496,11 +505,6 @@ int launch_get_aop(const aa_mie* t, int km, int nobs, int nch, int nq, const int
                        d_tracer_idx, d_chan_idx, d_qm, d_rh, nmom, npol, ntr_eff, normalize, d_tau, d_ssa, d_g,
                        d_pmom);
   };
-  // four moments per lane where rows, moments and the table base come in whole
-  // aligned groups of four and element offsets fit 32 bits
-  const long elems = (long)t->dev.ntracer * t->dev.nch * t->dev.nrh * t->dev.npol * t->dev.nmom;
-  const bool v4 = d_pmom && nmom % 4 == 0 && t->dev.nmom % 4 == 0 && ((size_t)t->dev.pmom & 15) == 0 &&
-                  elems <= 0x7fffffffL;
   if (!v4) launch(std::integral_constant<int, 0>());
   else if (mie_w4(nmom) == 8) launch(std::integral_constant<int, 8>());
   else if (mie_w4(nmom) == 16) launch(std::integral_constant<int, 16>());

@@ -28,3 +28,22 @@ def test_more_layer_chunks_than_a_grid_dimension(gpu, nmom):
     for a, b in zip(out[:4], ref[:4]):
         assert np.array_equal(a, b.T)
     assert out[4] == ref[4]
+
+
+@pytest.mark.parametrize("nmom,pairs", [(4, 24576), (4, 24577), (3, 49152), (3, 49153)])
+def test_chunks_apart_and_walked_are_the_same(gpu, nmom, pairs):
+    """Around the batch size from which a wavefront walks the layer chunks of its
+    column: the bits of a few columns by themselves."""
+    print(f"case chunks nmom={nmom} pairs={pairs}", flush=True)
+    km = 11
+    one = S.make_columns(97, km, CH, seed=47)
+    qm = np.resize(one.qm, (pairs,) + one.qm.shape[1:])
+    rh = np.resize(one.rh, (pairs, km))
+    mie = AM.MieTables.from_synthetic(S.make_mie_tables(CH, nmom=nmom, npol=1))
+    many = AM.get_aop_vector(mie, np.asarray(CH), S.TRACERS, 0, qm.T, rh.T, nmom, 1)
+    few = AM.get_aop_vector(mie, np.asarray(CH), S.TRACERS, 0, one.qm.T, one.rh.T, nmom, 1)
+    for a, b in zip(many[:4], few[:4]):
+        for lo in (0, 97 * (pairs // 97 - 1)):
+            assert np.array_equal(a[:, :, lo:lo + 97], b)
+        rest = pairs % 97
+        assert rest == 0 or np.array_equal(a[:, :, pairs - rest:], b[:, :, :rest])
